@@ -826,7 +826,9 @@ stereo_status stereo_crosscheck_configure(stereo_context* ctx, stereo_driver** o
     if ((st = driver_events(d))) return cleanup(st);
     if (injected_failure()) return cleanup(fail(ctx, STEREO_ERROR_HIP, "stereo_crosscheck_configure: injected failure"));
     hipError_t e;
-    if ((e = hipMalloc((void**)&d->range_dev, 2 * sizeof(uint32_t))) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipMalloc"));
+    if ((e = hipMalloc((void**)&d->range_dev, stereo::CROSSCHECK_STATE * sizeof(uint32_t))) != hipSuccess)
+        return cleanup(hip_fail(ctx, e, "hipMalloc"));
+    if ((e = stereo::crosscheck_state_init(d->range_dev)) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipMemcpy"));
     if ((e = hipHostMalloc((void**)&d->range_host, 2 * sizeof(uint32_t), 0)) != hipSuccess)
         return cleanup(hip_fail(ctx, e, "hipHostMalloc"));
     if ((e = hipEventCreateWithFlags(&d->ev_range, hipEventDisableTiming)) != hipSuccess)
@@ -859,10 +861,8 @@ stereo_status stereo_crosscheck_process(stereo_driver* d, stereo_image* result, 
     if ((st = begin(d, s))) return st;
     HIP_TRY(ctx,
             stereo::launch_crosscheck_ref(view_of(result), view_of(lr), view_of(rl), d->cc.disp_delta_thresh,
-                                          d->cc.left_to_right, d->cc.disp_offset, d->range_dev, s),
+                                          d->cc.left_to_right, d->cc.disp_offset, d->range_dev, d->range_host, s),
             "crosscheck launch");
-    HIP_TRY(ctx, hipMemcpyAsync(d->range_host, d->range_dev, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, s),
-            "hipMemcpyAsync");
     HIP_TRY(ctx, hipEventRecord(d->ev_range, s), "hipEventRecord");
     d->range_pending = true;
     return end(d, s);

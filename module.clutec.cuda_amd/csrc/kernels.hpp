@@ -142,9 +142,12 @@ hipError_t launch_bm_list_finish(const BmListParams& p, int max_width, hipStream
 constexpr int BM_LIST_MAX_WIDTH = BM_MAX_WIDTH;
 
 // ---- reference-format cross check ------------------------------------------------
-// range[0..1] receive min / max of the kept ids (device memory, reset by the launch).
+// state: CROSSCHECK_STATE device words, initialised once and left initialised by every launch;
+// result[0..1] (host memory the device can write) receive min / max of the kept ids.
+constexpr int CROSSCHECK_STATE = 3;
+hipError_t crosscheck_state_init(uint32_t* state);
 hipError_t launch_crosscheck_ref(const View& out, const View& lr, const View& rl, int thresh, int ltor, int offset,
-                                 uint32_t* range, hipStream_t s);
+                                 uint32_t* state, uint32_t* result, hipStream_t s);
 
 // ---- NCC matcher ------------------------------------------------------------------
 struct NccParams {

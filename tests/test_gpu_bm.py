@@ -176,6 +176,25 @@ def test_crosscheck_reference(ctx, ltor, thresh, offset):
     assert cc.range() == (mn, mx)
 
 
+@pytest.mark.parametrize("W,H", [(48, 1), (255, 3), (256, 16), (257, 17), (1021, 1100)])
+def test_crosscheck_segments_and_range(ctx, W, H):
+    """Row segments of 256 pixels, the last one ragged, fewer and more than one launch holds at once;
+    one driver over several frames: the range starts anew each time, also where nothing is kept."""
+    print(f"crosscheck {W}x{H}", flush=True)
+    rng = np.random.default_rng(W + H)
+    cc = cs.CrossCheck(ctx, W, H, thresh=1)
+    for frame, D in enumerate((200, 12, 0, 40)):
+        lr = _random_id_map(rng, W, H, max(D, 1))
+        rl = lr.copy()
+        rl[:, :, 0] = np.clip(lr[:, :, 0].astype(int) + rng.integers(-2, 3, (H, W)), 0, 65535)
+        if D == 0:
+            lr[:, :, 0] = orc.DISP_NOT_FOUND
+        got = cc.run(lr, rl)
+        ref, mn, mx = orc.crosscheck_ref(lr, rl, 1, 1, 0)
+        assert np.array_equal(got, ref), frame
+        assert cc.range() == (mn, mx), frame
+
+
 def test_crosscheck_format_mismatch(ctx):
     cc = cs.CrossCheck(ctx, 32, 16)
     a = cs.DeviceImage(ctx, 32, 16, cs.PIXEL_RGBA_U16)
