@@ -172,76 +172,190 @@ __global__ __launch_bounds__(256) void conv3x3_kernel(CnnConvArgs a)
 // Weight and bias gradients, one partial sum per workgroup:
 //   part[blk][(co*9 + t)*CIN + ci] = sum over the workgroup's pixels of dY[p][co] X[p+off_t][ci]
 //   part[blk][COUT*9*CIN + co]     = sum of dY[p][co]
-// Wave w of the workgroup owns the 16x16 block (co block w / KC, ci block w % KC).
-template <int CIN, int COUT>
-__global__ __launch_bounds__(256) void conv3x3_dw_kernel(CnnDwArgs a)
+// The pixels are the contraction (K), so an operand is four pixels of one channel, across
+// the NHWC layout.  A workgroup stages tiles of DW_ROWS rows x 64 pixels of both tensors in
+// LDS with the channel outermost, two pixels of a channel in one dword (v_perm_b32 pairs up
+// two 16-byte loads): an operand is then one 8-byte read, and the three horizontal taps of a
+// row come from one 12-pixel run of it by register shifts.  Wave w takes row w of the tile;
+// the waves' sums meet in LDS at the end.
+// What bounds it: the two tensors' bytes (33 MB for 16 frames of 240 x 135 at 16 channels) and
+// the LDS transpose; the MFMAs are 2 % of either.  The form it replaces read every operand
+// from global memory two bytes at a time on one wave per workgroup, 2 waves per CU: 163.8 us
+// at that size, against 20.7 / 23.0 / 28.5 us at dilation 1 / 2 / 4 (the rows of the halo, read
+// by the neighbouring tiles too, grow with the dilation).
+constexpr int DW_ROWS = 4;
+constexpr int DW_PX = 80;  // staged pixels of a row: x0 - 8 .. x0 + 71
+
+// Dwords between the channels of a staged tile of `rows` rows: 8 mod 32, so that the 16
+// channels x 4 pixel groups of an operand read fall in 32 different banks twice over.
+constexpr int dw_stride(int rows, int px) { return ((rows * px / 2 + 23) & ~31) + 8; }
+
+// rows x (64 + 2 PAD) pixels of the NHWC image at (x0 - PAD, ytop), zero outside it, to LDS.
+template <int C, int ROWS, int PAD>
+__device__ __forceinline__ void dw_stage(uint32_t* dst, const uint16_t* img, int W, int H, int x0, int ytop)
 {
-    constexpr int KC = CIN / 16, MB = COUT / 16;
-    const int lane = threadIdx.x & 63;
-    const int col = lane & 15, grp = lane >> 4;
-    const int w = threadIdx.x >> 6;
-    if (w >= MB * KC) return;
-    const int mb = w / KC, kb = w % KC;
-    const int co = mb * 16 + col;  // A row of this lane
-    const int ci = kb * 16 + col;  // B column of this lane
-    v4f acc[9];
-#pragma unroll
-    for (int t = 0; t < 9; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-    float bsum = 0.f;
-    const int nbx = (a.W + 15) >> 4;
-    const int total = a.N * a.H * nbx;
-    for (int b = blockIdx.x; b < total; b += gridDim.x) {
-        const int bxi = b % nbx;
-        const int r = b / nbx;
-        const int yy = r % a.H;
-        const int n = r / a.H;
-        const int p0 = bxi * 16 + 4 * grp;
-        v4s av;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int px = p0 + i;
-            const bool ok = px < a.W;
-            const size_t idx = ok ? (((size_t)n * a.H + yy) * a.W + px) * COUT + co : 0;  // in-bounds address
-            const uint16_t g = ok ? a.dy[idx] : (uint16_t)0;
-            av[i] = (short)g;
-            bsum += bf2f(g);
+    constexpr int PAIRS = 32 + PAD, QP = C / 8, N = ROWS * PAIRS * QP, CS = dw_stride(ROWS, 64 + 2 * PAD);
+    for (int i = threadIdx.x; i < N; i += 256) {
+        const int q = i % QP, k = i / QP;
+        const int pp = k % PAIRS, r = k / PAIRS;
+        const int x = x0 - PAD + 2 * pp, y = ytop + r;
+        uint4 a = make_uint4(0u, 0u, 0u, 0u), b = a;
+        if (y >= 0 && y < H) {
+            const uint16_t* p = img + ((ptrdiff_t)y * W + x) * C + 8 * q;
+            if (x >= 0 && x < W) a = *reinterpret_cast<const uint4*>(p);
+            if (x + 1 >= 0 && x + 1 < W) b = *reinterpret_cast<const uint4*>(p + C);
         }
+        uint32_t* d = dst + (8 * q) * CS + r * PAIRS + pp;
+        const uint32_t av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
-        for (int t = 0; t < 9; ++t) {
-            const int sy = yy + (t / 3 - 1) * a.dil;
-            const bool rok = sy >= 0 && sy < a.H;
-            v4s bv;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int sx = p0 + i + (t % 3 - 1) * a.dil;
-                const bool ok = rok && sx >= 0 && sx < a.W && p0 + i < a.W;
-                const size_t idx = ok ? (((size_t)n * a.H + sy) * a.W + sx) * CIN + ci : 0;
-                const short v = (short)a.x[idx];
-                bv[i] = ok ? v : (short)0;
-            }
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[t], 0, 0, 0);
+        for (int j = 0; j < 4; ++j) {
+            d[(2 * j) * CS] = __builtin_amdgcn_perm(bv[j], av[j], 0x05040100u);
+            d[(2 * j + 1) * CS] = __builtin_amdgcn_perm(bv[j], av[j], 0x07060302u);
         }
-    }
-    float* part = a.part + (size_t)blockIdx.x * (COUT * 9 * CIN + COUT);
-    // D[m][n]: lane (col, grp) holds m = 4 grp + i (co), n = col (ci)
-#pragma unroll
-    for (int t = 0; t < 9; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) part[((mb * 16 + 4 * grp + i) * 9 + t) * CIN + kb * 16 + col] = acc[t][i];
-    if (kb == 0) {
-        bsum += __shfl_xor(bsum, 16);
-        bsum += __shfl_xor(bsum, 32);
-        if (grp == 0) part[COUT * 9 * CIN + co] = bsum;
     }
 }
 
-__global__ __launch_bounds__(256) void reduce_parts_kernel(const float* part, int nparts, int n, float* out)
+// LDS dwords of one workgroup: both staged tiles, and at the end one set of sums
+template <int CIN, int COUT, int DIL>
+constexpr int dw_lds()
 {
-    const int j = blockIdx.x * 256 + threadIdx.x;
-    if (j >= n) return;
+    constexpr int tiles = CIN * dw_stride(DW_ROWS + 2 * DIL, DW_PX) + COUT * dw_stride(DW_ROWS, 64);
+    constexpr int sums = COUT * 9 * CIN + COUT;
+    return tiles > sums ? tiles : sums;
+}
+
+template <int CIN, int COUT, int DIL>
+__global__ __launch_bounds__(256) void conv3x3_dw_kernel(CnnDwArgs a)
+{
+    constexpr int KC = CIN / 16, MB = COUT / 16;
+    constexpr int XR = DW_ROWS + 2 * DIL, XS = dw_stride(XR, DW_PX), GS = dw_stride(DW_ROWS, 64);
+    __shared__ __align__(16) uint32_t dw_tile[dw_lds<CIN, COUT, DIL>()];
+    uint32_t* const xs = dw_tile;
+    uint32_t* const gs = dw_tile + CIN * XS;
+    const int lane = threadIdx.x & 63;
+    const int col = lane & 15, grp = lane >> 4;
+    const int wv = threadIdx.x >> 6;
+    v4f acc[MB][KC][9];
+    float bsum[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        bsum[mb] = 0.f;
+#pragma unroll
+        for (int kb = 0; kb < KC; ++kb)
+#pragma unroll
+            for (int t = 0; t < 9; ++t) acc[mb][kb][t] = v4f{0.f, 0.f, 0.f, 0.f};
+    }
+    const int ntx = (a.W + 63) >> 6, nty = (a.H + DW_ROWS - 1) / DW_ROWS;
+    const int total = a.N * nty * ntx;
+    for (int b = blockIdx.x; b < total; b += gridDim.x) {
+        const int tx = b % ntx, r = b / ntx;
+        const int ty = r % nty, n = r / nty;
+        const int x0 = tx * 64, y0 = ty * DW_ROWS;
+        const size_t frame = (size_t)n * a.H * a.W;
+        __syncthreads();  // the previous tile's operands have been read
+        dw_stage<CIN, XR, 8>(xs, a.x + frame * CIN, a.W, a.H, x0, y0 - DIL);
+        dw_stage<COUT, DW_ROWS, 0>(gs, a.dy + frame * COUT, a.W, a.H, x0, y0);
+        __syncthreads();
+        for (int kb = 0; kb < 4; ++kb) {
+            const int px = 16 * kb + 4 * grp;  // this lane's four pixels of the row
+            v4s av[MB];
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+                const uint2 g = *reinterpret_cast<const uint2*>(gs + (mb * 16 + col) * GS + wv * 32 + px / 2);
+                av[mb] = __builtin_bit_cast(v4s, g);
+                bsum[mb] += (bf2f(g.x) + bf2f(g.x >> 16)) + (bf2f(g.y) + bf2f(g.y >> 16));
+            }
+            // pixels past the image: their gradient is 0 and must meet 0, whatever X holds
+            const int in = a.W - (x0 + px);
+            const uint32_t m0 = in >= 2 ? ~0u : (in == 1 ? 0xFFFFu : 0u), m1 = in >= 4 ? ~0u : (in == 3 ? 0xFFFFu : 0u);
+#pragma unroll
+            for (int ky = 0; ky < 3; ++ky)
+#pragma unroll
+                for (int kc = 0; kc < KC; ++kc) {
+                    const uint32_t* src = xs + (kc * 16 + col) * XS + (wv + ky * DIL) * (DW_PX / 2) + (px + 4) / 2;
+                    uint32_t v[6];  // pixels px - 4 .. px + 7
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        const uint2 q = *reinterpret_cast<const uint2*>(src + 2 * k);
+                        v[2 * k] = q.x;
+                        v[2 * k + 1] = q.y;
+                    }
+#pragma unroll
+                    for (int kx = 0; kx < 3; ++kx) {
+                        constexpr int odd = DIL & 1;
+                        const int s = 4 + (kx - 1) * DIL, w = s >> 1;
+                        const bool shift = kx != 1 && odd;
+                        uint2 x;
+                        x.x = (shift ? __builtin_amdgcn_alignbit(v[w + 1 < 6 ? w + 1 : 5], v[w], 16) : v[w]) & m0;
+                        x.y = (shift ? __builtin_amdgcn_alignbit(v[w + 2 < 6 ? w + 2 : 5], v[w + 1], 16) : v[w + 1]) & m1;
+#pragma unroll
+                        for (int mb = 0; mb < MB; ++mb)
+                            acc[mb][kc][3 * ky + kx] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                                av[mb], __builtin_bit_cast(v4s, x), acc[mb][kc][3 * ky + kx], 0, 0, 0);
+                    }
+                }
+        }
+    }
+    // the four waves' sums, in wave order, in the layout of the partial sum
+    constexpr int NS = COUT * 9 * CIN + COUT;
+    float* const sums = reinterpret_cast<float*>(dw_tile);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        bsum[mb] += __shfl_xor(bsum[mb], 16);
+        bsum[mb] += __shfl_xor(bsum[mb], 32);
+    }
+    for (int w = 0; w < 4; ++w) {
+        __syncthreads();
+        if (wv != w) continue;
+        // D[m][n]: lane (col, grp) holds m = 4 grp + i (co), n = col (ci)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+                for (int t = 0; t < 9; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        float* p = sums + ((mb * 16 + 4 * grp + i) * 9 + t) * CIN + kc * 16 + col;
+                        *p = w ? *p + acc[mb][kc][t][i] : acc[mb][kc][t][i];
+                    }
+            if (grp == 0) {
+                float* p = sums + COUT * 9 * CIN + mb * 16 + col;
+                *p = w ? *p + bsum[mb] : bsum[mb];
+            }
+        }
+    }
+    __syncthreads();
+    float* part = a.part + (size_t)blockIdx.x * NS;
+    for (int i = threadIdx.x; i < NS; i += 256) part[i] = sums[i];
+}
+
+// Adds the partial sums of 16 values per workgroup, 16 threads to a value, in a fixed order.
+// One thread per value read its nparts dependent loads one after another: 119.8 us for 512
+// partial sums of 2320 values, against 4.8 us for 436 of them.
+constexpr int RED_V = 16, RED_G = 16;
+
+__device__ __forceinline__ float reduce_part(const float* part, int nparts, int n, int j, int g, float (*red)[RED_V + 1])
+{
     float s = 0.f;
-    for (int b = 0; b < nparts; ++b) s += part[(size_t)b * n + j];
-    out[j] = s;
+    if (j < n) {
+#pragma unroll 8
+        for (int b = g; b < nparts; b += RED_G) s += part[(size_t)b * n + j];
+    }
+    red[g][threadIdx.x & (RED_V - 1)] = s;
+    __syncthreads();
+    s = 0.f;
+    if (g == 0)
+        for (int k = 0; k < RED_G; ++k) s += red[k][threadIdx.x & (RED_V - 1)];
+    return s;
+}
+
+__global__ __launch_bounds__(RED_V * RED_G) void reduce_parts_kernel(const float* part, int nparts, int n, float* out)
+{
+    __shared__ float red[RED_G][RED_V + 1];
+    const int j = blockIdx.x * RED_V + (threadIdx.x & (RED_V - 1)), g = threadIdx.x / RED_V;
+    const float s = reduce_part(part, nparts, n, j, g, red);
+    if (g == 0 && j < n) out[j] = s;
 }
 
 // Loss over the network output (FP32, 16 channels; channel 0 = centre residual in
@@ -723,27 +837,53 @@ hipError_t launch_cnn_conv(int cin, int cout, int epi, const CnnConvArgs& a, hip
     return hipErrorInvalidValue;
 }
 
+// Workgroups of the weight gradient: two per CU, every one with the same number of tiles (the
+// last few one less), and each leaves one partial sum.
 int cnn_dw_parts(const CnnDwArgs& a)
 {
-    const long total = (long)a.N * a.H * ((a.W + 15) / 16);
-    long g = (total + 7) / 8;
-    if (g > 512) g = 512;
-    if (g < 1) g = 1;
-    return (int)g;
+    const long total = (long)a.N * ((a.H + cnn::DW_ROWS - 1) / cnn::DW_ROWS) * ((a.W + 63) / 64);
+    const long each = (total + 511) / 512;
+    const long g = (total + each - 1) / each;
+    return g < 1 ? 1 : (int)g;
+}
+
+int cnn_dw_max_parts(const CnnDwArgs& a)
+{
+    const long total = (long)a.N * ((a.H + cnn::DW_ROWS - 1) / cnn::DW_ROWS) * ((a.W + 63) / 64);
+    return total < 1 ? 1 : (total > 512 ? 512 : (int)total);
+}
+
+template <int CI, int CO, int DIL>
+static hipError_t launch_dw(const CnnDwArgs& a, int grid, hipStream_t s)
+{
+    hipLaunchKernelGGL((cnn::conv3x3_dw_kernel<CI, CO, DIL>), dim3(grid), dim3(256), 0, s, a);
+    return hipGetLastError();
 }
 
 hipError_t launch_cnn_dw(int cin, int cout, const CnnDwArgs& a, float* out, hipStream_t s)
 {
+    if (a.N < 1 || a.H < 1 || a.W < 1 || a.dil < 1 || a.dil > CNN_MAX_DIL) return hipErrorInvalidValue;
+    if ((long)a.N * ((a.H + cnn::DW_ROWS - 1) / cnn::DW_ROWS) * ((a.W + 63) / 64) > 0x3fffffffL) return hipErrorInvalidValue;
     const int grid = cnn_dw_parts(a);
-    if (cin == 16 && cout == 16) hipLaunchKernelGGL((cnn::conv3x3_dw_kernel<16, 16>), dim3(grid), dim3(256), 0, s, a);
-    else if (cin == 16 && cout == 32) hipLaunchKernelGGL((cnn::conv3x3_dw_kernel<16, 32>), dim3(grid), dim3(256), 0, s, a);
-    else if (cin == 32 && cout == 32) hipLaunchKernelGGL((cnn::conv3x3_dw_kernel<32, 32>), dim3(grid), dim3(256), 0, s, a);
-    else if (cin == 32 && cout == 16) hipLaunchKernelGGL((cnn::conv3x3_dw_kernel<32, 16>), dim3(grid), dim3(256), 0, s, a);
-    else return hipErrorInvalidValue;
-    hipError_t e = hipGetLastError();
+    hipError_t e = hipErrorInvalidValue;
+#define CNN_DW(CI, CO)                                          \
+    if (cin == CI && cout == CO) {                              \
+        switch (a.dil) {                                        \
+        case 1: e = launch_dw<CI, CO, 1>(a, grid, s); break;    \
+        case 2: e = launch_dw<CI, CO, 2>(a, grid, s); break;    \
+        case 3: e = launch_dw<CI, CO, 3>(a, grid, s); break;    \
+        default: e = launch_dw<CI, CO, 4>(a, grid, s); break;   \
+        }                                                       \
+    }
+    CNN_DW(16, 16)
+    CNN_DW(16, 32)
+    CNN_DW(32, 32)
+    CNN_DW(32, 16)
+#undef CNN_DW
     if (e != hipSuccess) return e;
     const int n = cout * 9 * cin + cout;
-    hipLaunchKernelGGL(cnn::reduce_parts_kernel, dim3((n + 255) / 256), dim3(256), 0, s, (const float*)a.part, grid, n, out);
+    hipLaunchKernelGGL(cnn::reduce_parts_kernel, dim3((n + cnn::RED_V - 1) / cnn::RED_V), dim3(cnn::RED_V * cnn::RED_G), 0, s,
+                       (const float*)a.part, grid, n, out);
     return hipGetLastError();
 }
 

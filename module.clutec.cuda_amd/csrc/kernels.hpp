@@ -248,6 +248,7 @@ struct CnnFusedArgs {
 };
 hipError_t launch_cnn_fused_forward(const CnnFusedArgs& a, hipStream_t s);
 int cnn_dw_parts(const CnnDwArgs& a);
+int cnn_dw_max_parts(const CnnDwArgs& a);  // the most parts of any a.N up to this one
 hipError_t launch_cnn_dw(int cin, int cout, const CnnDwArgs& a, float* out, hipStream_t s);
 // clabel: per-pixel confidence target (0 or 1, NaN: from |e| <= tau where label is set)
 hipError_t launch_cnn_loss(const float* out, const float* label, const float* clabel, const float* dfill, uint16_t* g,

@@ -208,8 +208,8 @@ stereo_status stereo_cnn_create(stereo_context* ctx, stereo_cnn** out, int32_t W
     da.N = max_frames;
     da.H = H4;
     da.W = W4;
-    c->dwparts = stereo::cnn_dw_parts(da);
-    if ((e = hipMalloc((void**)&c->dwpart, (size_t)c->dwparts * (32 * 9 * 32 + 32) * 4))) return bail(e);
+    c->dwparts = stereo::cnn_dw_max_parts(da);
+    if ((e = hipMalloc((void**)&c->dwpart, (size_t)c->dwparts * layer_n(0) * 4))) return bail(e);
     if ((e = hipMemset(c->param, 0, np * 4)) || (e = hipMemset(c->grad, 0, np * 4)) || (e = hipMemset(c->m, 0, np * 4)) ||
         (e = hipMemset(c->v, 0, np * 4)) || (e = hipMemset(c->labels, 0xFF, P * 4)) ||
         (e = hipMemset(c->clabels, 0xFF, P * 4)) || (e = hipMemset(c->dfill, 0, P * 4)) ||
