@@ -366,45 +366,6 @@ __global__ __launch_bounds__(256, Cost::LIST_WG) void bm_list_kernel(BmListParam
     }
 }
 
-// TPS: the most tiles a segment's left pixels xr + ds .. xr + de - 1 can span,
-// (seg_len - 1) / 64 + 2, at most 5 (seg_len <= 256).
-template <int TPS>
-__device__ __forceinline__ uint32_t rkey_at(const BmFinishParams& f, int xr, int y)
-{
-    // right pixel xr meets left pixels xr+d; segment s covers d in [ds, de), and the
-    // tile holding left pixel x keeps the partial under index xr - x0 + 255.  A
-    // segment spans at most TPS tiles.  Two segments' loads are issued
-    // together and unconditionally: past the segment's last tile a load repeats that
-    // tile (the max is unchanged), and a segment with no tile reads a fixed address
-    // whose value is discarded.
-    uint32_t best = 0;
-    for (int s0 = 0; s0 < f.nseg; s0 += 2) {
-        uint32_t v[2][TPS];
-        bool any[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int s = min(s0 + q, f.nseg - 1);
-            const int ds = s * f.seg_len;
-            const int de = min(f.D, ds + f.seg_len);
-            const int tlo = (xr + ds) / 64;
-            const int thi = min((xr + de - 1) / 64, f.ntx - 1);
-            any[q] = tlo <= thi;
-            const uint32_t* base = f.rpart + ((size_t)s * f.ntx * f.H + y) * BM_NPART + (xr + 255);
-#pragma unroll
-            for (int j = 0; j < TPS; ++j) {
-                const int t = min(tlo + j, thi);
-                const uint32_t* a = any[q] ? base + ((size_t)t * f.H * BM_NPART - 64 * t) : f.rpart;
-                v[q][j] = *a;
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int j = 0; j < TPS; ++j) best = (any[q] && v[q][j] > best) ? v[q][j] : best;
-    }
-    return best;
-}
-
 // Output of one left pixel: the checked disparity and the maps, in every requested
 // format.  lk = merged left key, rrow = merged right keys of the row.
 __device__ __forceinline__ void write_pixel(const View& disp, const View& disp_l, const View& disp_r,
@@ -440,99 +401,37 @@ __device__ __forceinline__ void write_pixel(const View& disp, const View& disp_l
     }
 }
 
-// One workgroup per image row: first every right pixel of the row merges its partial
-// keys (contiguous reads, one pass) into LDS, then every left pixel looks up the right
-// winner at x - dL for the check.  The left keys of a thread's first FIN_PF pixels are
-// loaded before the barrier, so their latency overlaps the right-key merge.
+// One workgroup per image row.  The left keys of a thread's first FIN_PF pixels are loaded
+// before the barrier, so their latency overlaps the right keys' pass.
 constexpr int FIN_PF = 8;
-
-__device__ __forceinline__ uint32_t lkey_at(const BmFinishParams& f, int x, int y)
-{
-    uint32_t lk = 0;
-    for (int s = 0; s < f.nseg; ++s) {
-        const uint32_t v = f.lkey[(size_t)s * f.W * f.H + (size_t)y * f.W + x];
-        lk = v > lk ? v : lk;
-    }
-    return lk;
-}
-
-template <int TPS>
-__global__ __launch_bounds__(256) void bm_finish_kernel(BmFinishParams f)
-{
-    extern __shared__ uint32_t rrow[];
-    const int y = blockIdx.x;
-    const int W = f.W;
-    const bool row_ok = y >= f.by && y < f.H - f.by;
-    // the left keys of the thread's first FIN_PF pixels, two segments per batch of loads
-    // (a position past the row reads the row's last pixel; the value is discarded;
-    // slots wholly past the row are skipped)
-    uint32_t lpre[FIN_PF];
-    {
-        const size_t plane = (size_t)W * f.H;
-#pragma unroll
-        for (int k = 0; k < FIN_PF; ++k) lpre[k] = 0u;
-        for (int s0 = 0; s0 < f.nseg; s0 += 2) {
-            const size_t sa = (size_t)s0 * plane, sb = (size_t)min(s0 + 1, f.nseg - 1) * plane;
-            uint32_t la[FIN_PF], lb[FIN_PF];
-#pragma unroll
-            for (int k = 0; k < FIN_PF; ++k) {
-                la[k] = lb[k] = 0u;
-                if (256 * k < W) {
-                    const size_t i = (size_t)y * W + min((int)threadIdx.x + 256 * k, W - 1);
-                    la[k] = f.lkey[sa + i];
-                    lb[k] = f.lkey[sb + i];
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < FIN_PF; ++k) {
-                const uint32_t m = la[k] > lb[k] ? la[k] : lb[k];
-                lpre[k] = m > lpre[k] ? m : lpre[k];
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < FIN_PF; ++k) {
-            const int x = threadIdx.x + 256 * k;
-            if (!(row_ok && x >= f.bx && x < W - f.bx)) lpre[k] = 0u;
-        }
-    }
-#pragma unroll 2
-    for (int x = threadIdx.x; x < W; x += 256) {
-        const bool col_ok = x >= f.bx && x < W - f.bx;
-        const uint32_t r = rkey_at<TPS>(f, x, y);
-        rrow[x] = (row_ok && col_ok) ? r : 0u;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < FIN_PF; ++k) {
-        const int x = threadIdx.x + 256 * k;
-        if (x < W)
-            write_pixel(f.disp, f.disp_l, f.disp_r, f.dispid, x, y, row_ok && x >= f.bx && x < W - f.bx, lpre[k], rrow,
-                        f.tol, f.value_base);
-    }
-    for (int x = threadIdx.x + 256 * FIN_PF; x < W; x += 256) {
-        const bool inside = row_ok && x >= f.bx && x < W - f.bx;
-        write_pixel(f.disp, f.disp_l, f.disp_r, f.dispid, x, y, inside, inside ? lkey_at(f, x, y) : 0u, rrow, f.tol,
-                    f.value_base);
-    }
-}
 
 // Check of one image row from the key planes that the matchers fold their keys into
 // with atomicMax: the workgroup reads the row's right keys into LDS and every left pixel
 // looks up the right winner at x - dL.  Each key is cleared by the thread that read it,
-// so the planes start the next frame at zero.
+// so the planes start the next frame at zero.  KEEP: the left keys are nlseg segments, lseg
+// elements apart, and stay.
+template <bool KEEP>
 __device__ __forceinline__ void planes_row(const View& disp, const View& disp_l, const View& disp_r, const View& dispid,
                                            int W, int y, bool row_ok, int bx, int tol, int value_base, uint32_t* lrow,
-                                           uint32_t* rrowg, uint32_t* rrow)
+                                           uint32_t* rrowg, uint32_t* rrow, int nlseg = 1, size_t lseg = 0)
 {
+    auto left_key = [&](int x) {
+        uint32_t k = lrow[x];
+        if (KEEP) {
+            for (int s = 1; s < nlseg; ++s) {
+                const uint32_t v = lrow[(size_t)s * lseg + x];
+                k = v > k ? v : k;
+            }
+        } else {
+            lrow[x] = 0u;
+        }
+        return k;
+    };
     uint32_t lpre[FIN_PF];
 #pragma unroll
     for (int k = 0; k < FIN_PF; ++k) {
         const int x = threadIdx.x + 256 * k;
-        lpre[k] = 0u;
-        if (x < W) {
-            lpre[k] = lrow[x];
-            lrow[x] = 0u;
-        }
+        lpre[k] = x < W ? left_key(x) : 0u;
     }
     for (int x = threadIdx.x; x < W; x += 256) {
         const bool col_ok = x >= bx && x < W - bx;
@@ -551,21 +450,21 @@ __device__ __forceinline__ void planes_row(const View& disp, const View& disp_l,
     }
     for (int x = threadIdx.x + 256 * FIN_PF; x < W; x += 256) {
         const bool inside = row_ok && x >= bx && x < W - bx;
-        const uint32_t lk = lrow[x];
-        lrow[x] = 0u;
+        const uint32_t lk = left_key(x);
         write_pixel(disp, disp_l, disp_r, dispid, x, y, inside, inside ? lk : 0u, rrow, tol, value_base);
     }
 }
 
-// SAD / census grid launch: one workgroup per image row.
+// Grid launch: one workgroup per image row.
+template <bool KEEP>
 __global__ __launch_bounds__(256) void bm_finish_planes_kernel(BmFinishParams f)
 {
     extern __shared__ uint32_t rrow[];
     const int y = blockIdx.x;
     const bool row_ok = y >= f.by && y < f.H - f.by;
-    planes_row(f.disp, f.disp_l, f.disp_r, f.dispid, f.W, y, row_ok, f.bx, f.tol, f.value_base,
-               f.lplane + (size_t)y * f.W, f.rplane + (size_t)y * f.W, rrow);
-    if (f.cnn.x) {
+    planes_row<KEEP>(f.disp, f.disp_l, f.disp_r, f.dispid, f.W, y, row_ok, f.bx, f.tol, f.value_base,
+                     f.lplane + (size_t)y * f.W, f.rplane + (size_t)y * f.W, rrow, f.nlseg, (size_t)f.W * f.H);
+    if (!KEEP && f.cnn.x) {
         // the learned proposal's network input from the row just written
         __shared__ uint64_t valid[CNN_MAX_W4 / 64];
         __syncthreads();
@@ -601,8 +500,8 @@ __global__ __launch_bounds__(256) void bm_list_finish_kernel(BmListParams p)
     const int y = r - f.row_base;
     const bool row_ok = y >= f.by && y < f.H - f.by;
     const size_t row = f.plane_off + (size_t)y * f.W;
-    planes_row(f.disp, f.disp_l, f.disp_r, f.dispid, f.W, y, row_ok, f.bx, f.tol, f.value_base, p.lplane + row,
-               p.rplane + row, rrow);
+    planes_row<false>(f.disp, f.disp_l, f.disp_r, f.dispid, f.W, y, row_ok, f.bx, f.tol, f.value_base, p.lplane + row,
+                      p.rplane + row, rrow);
 }
 
 }  // namespace bm
@@ -684,21 +583,15 @@ hipError_t launch_bm_clear(uint32_t* p, size_t n, hipStream_t s)
 
 hipError_t launch_bm_finish(const BmFinishParams& f, hipStream_t s)
 {
-    if (f.W > BM_MAX_WIDTH || f.seg_len < 1 || f.seg_len > 256) return hipErrorInvalidValue;
+    if (f.W > BM_MAX_WIDTH || !f.lplane || !f.rplane) return hipErrorInvalidValue;
     const size_t lds = (size_t)f.W * sizeof(uint32_t);
-    if (f.lplane) {
-        if (!f.rplane) return hipErrorInvalidValue;
-        if (f.cnn.x && (!f.disp.ptr || !f.cnn.dfill || f.W > CNN_MAX_W4 || f.cnn.L4.w != f.W || f.cnn.L4.h != f.H ||
-                        f.cnn.R4.w != f.W || f.cnn.R4.h != f.H))
-            return hipErrorInvalidValue;
-        hipLaunchKernelGGL(bm::bm_finish_planes_kernel, dim3(f.H), dim3(256), lds, s, f);
-        return hipGetLastError();
-    }
-    const int tps = (f.seg_len - 1) / bm::TW + 2;
-    if (tps <= 2) hipLaunchKernelGGL(bm::bm_finish_kernel<2>, dim3(f.H), dim3(256), lds, s, f);
-    else if (tps == 3) hipLaunchKernelGGL(bm::bm_finish_kernel<3>, dim3(f.H), dim3(256), lds, s, f);
-    else if (tps == 4) hipLaunchKernelGGL(bm::bm_finish_kernel<4>, dim3(f.H), dim3(256), lds, s, f);
-    else hipLaunchKernelGGL(bm::bm_finish_kernel<5>, dim3(f.H), dim3(256), lds, s, f);
+    if (f.cnn.x && (f.nlseg || !f.disp.ptr || !f.cnn.dfill || f.W > CNN_MAX_W4 || f.cnn.L4.w != f.W || f.cnn.L4.h != f.H ||
+                    f.cnn.R4.w != f.W || f.cnn.R4.h != f.H))
+        return hipErrorInvalidValue;
+    if (f.nlseg)
+        hipLaunchKernelGGL(bm::bm_finish_planes_kernel<true>, dim3(f.H), dim3(256), lds, s, f);
+    else
+        hipLaunchKernelGGL(bm::bm_finish_planes_kernel<false>, dim3(f.H), dim3(256), lds, s, f);
     return hipGetLastError();
 }
 

@@ -449,7 +449,7 @@ stereo_status stereo_matcher_configure(stereo_context* ctx, stereo_driver** out,
     d->by = p->window_h / 2 + (census ? p->census_h / 2 : 0);
     if (aw) d->bx = d->by = p->window_w + p->window_w / 2;
     if (ncc)
-        stereo::ncc_grid(fmt->width, fmt->height, p->num_disparities, &d->ntx, &d->nty, &d->nseg, &d->seg_len);
+        stereo::ncc_grid(fmt->width, fmt->height, p->num_disparities, &d->ntx, &d->rb, &d->nseg, &d->seg_len);
     else if (aw)
         stereo::aw_grid(fmt->width, fmt->height, p->num_disparities, &d->ntx, &d->nty, &d->nseg, &d->seg_len);
     else
@@ -462,29 +462,28 @@ stereo_status stereo_matcher_configure(stereo_context* ctx, stereo_driver** out,
     if ((st = driver_events(d))) return cleanup(st);
     if (injected_failure()) return cleanup(fail(ctx, STEREO_ERROR_HIP, "stereo_matcher_configure: injected failure"));
     hipError_t e;
-    if ((e = hipMalloc((void**)&d->padL, d->pad_pitch * H)) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipMalloc"));
-    if ((e = hipMalloc((void**)&d->padR, d->pad_pitch * H)) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipMalloc"));
+    // NCC reads the images themselves, and keeps a left key plane per disparity segment
+    const size_t lplanes = ncc ? d->nseg : 1, nstats = W * H + stereo::NCC_STATS_PAD;
+    if (!ncc && ((e = hipMalloc((void**)&d->padL, d->pad_pitch * H)) || (e = hipMalloc((void**)&d->padR, d->pad_pitch * H))))
+        return cleanup(hip_fail(ctx, e, "hipMalloc"));
+    // the key planes start at zero; every frame's merge leaves them so
+    if ((e = hipMalloc((void**)&d->lkey, lplanes * W * H * 4)) || (e = hipMalloc((void**)&d->rkey, W * H * 4)))
+        return cleanup(hip_fail(ctx, e, "hipMalloc"));
+    if ((e = hipMemset(d->lkey, 0, lplanes * W * H * 4)) || (e = hipMemset(d->rkey, 0, W * H * 4)))
+        return cleanup(hip_fail(ctx, e, "hipMemset"));
     if (ncc) {
-        // per segment: stereo_matcher_scores reads the left keys after the frame
-        if ((e = hipMalloc((void**)&d->lkey, (size_t)d->nseg * W * H * 4)) != hipSuccess)
+        if ((e = hipMalloc((void**)&d->lstats, nstats * sizeof(int2))) || (e = hipMalloc((void**)&d->rstats, nstats * sizeof(int2))))
             return cleanup(hip_fail(ctx, e, "hipMalloc"));
-        if ((e = hipMalloc((void**)&d->rpart, (size_t)d->nseg * d->ntx * H * stereo::BM_NPART * 4)) != hipSuccess)
-            return cleanup(hip_fail(ctx, e, "hipMalloc"));
+        // the pad past the last pixel is read for blocks at the right edge, and masked
+        if ((e = hipMemset(d->lstats + W * H, 0, stereo::NCC_STATS_PAD * sizeof(int2))) ||
+            (e = hipMemset(d->rstats + W * H, 0, stereo::NCC_STATS_PAD * sizeof(int2))))
+            return cleanup(hip_fail(ctx, e, "hipMemset"));
     } else {
-        // the key planes start at zero; every frame's merge leaves them so
-        if ((e = hipMalloc((void**)&d->lkey, W * H * 4)) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipMalloc"));
-        if ((e = hipMalloc((void**)&d->rkey, W * H * 4)) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipMalloc"));
-        if ((e = hipMemset(d->lkey, 0, W * H * 4)) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipMemset"));
-        if ((e = hipMemset(d->rkey, 0, W * H * 4)) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipMemset"));
+        // the pad columns only ever meet masked candidates; clear them once so that no
+        // uninitialised memory is read
+        if ((e = hipMemset(d->padL, 0, d->pad_pitch * H)) || (e = hipMemset(d->padR, 0, d->pad_pitch * H)))
+            return cleanup(hip_fail(ctx, e, "hipMemset"));
     }
-    if (ncc) {
-        if ((e = hipMalloc((void**)&d->lstats, W * H * sizeof(int2))) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipMalloc"));
-        if ((e = hipMalloc((void**)&d->rstats, W * H * sizeof(int2))) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipMalloc"));
-    }
-    // the pad columns only ever meet masked candidates; clear them once so that no
-    // uninitialised memory is read
-    if ((e = hipMemset(d->padL, 0, d->pad_pitch * H)) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipMemset"));
-    if ((e = hipMemset(d->padR, 0, d->pad_pitch * H)) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipMemset"));
     if (p->use_disp_input && (st = band_alloc(d))) return cleanup(st);
     *out = d;
     return STEREO_OK;
@@ -503,42 +502,48 @@ static stereo_status matcher_run(stereo_driver* d, stereo_image* disp, bool disp
     pl.pitch = pr.pitch = d->pad_pitch;
     pl.w = pr.w = W;
     pl.h = pr.h = H;
-    pl.ptr = d->padL + (size_t)stereo::BM_PAD_LEFT * d->pad_elem;
-    pr.ptr = d->padR + (size_t)stereo::BM_PAD_LEFT * d->pad_elem;
+    pl.ptr = d->padL ? d->padL + (size_t)stereo::BM_PAD_LEFT * d->pad_elem : nullptr;
+    pr.ptr = d->padR ? d->padR + (size_t)stereo::BM_PAD_LEFT * d->pad_elem : nullptr;
     const bool census = d->mp.algorithm == STEREO_ALGO_CENSUS;
     const bool ncc = d->mp.algorithm == STEREO_ALGO_NCC;
     const bool aw = d->mp.algorithm == STEREO_ALGO_AW1 || d->mp.algorithm == STEREO_ALGO_AW2;
     if (census) {
         const View vl = view_of(left), vr = view_of(right);
         HIP_TRY(ctx, stereo::launch_census_pair(vl, pl, &vr, &pr, d->mp.census_w, d->mp.census_h, s), "census launch");
+    } else if (ncc) {
+        HIP_TRY(ctx, stereo::launch_ncc_stats_pair(view_of(left), d->lstats, 8388608.0f, view_of(right), d->rstats, 1.0f, W,
+                                                   d->mp.window_w, s),
+                "ncc stats launch");
     } else {
         HIP_TRY(ctx, stereo::launch_pad_copy_pair(view_of(left), pl, view_of(right), pr, s), "copy launch");
     }
-    if (ncc) {
-        HIP_TRY(ctx, stereo::launch_ncc_stats_pair(view_of(left), d->lstats, 8388608.0f, view_of(right), d->rstats, 1.0f, W,
-                                                   d->mp.window_w, d->mp.window_h, s),
-                "ncc stats launch");
-    }
     if (ctx->timing) HIP_TRY(ctx, hipEventRecord(d->ev_stage[0], s), "hipEventRecord");
     if (ncc) {
+        if (d->planes_dirty) {
+            // an earlier frame's merge did not run: clear what its matcher folded in
+            HIP_TRY(ctx, stereo::launch_bm_clear(d->rkey, (size_t)W * H, s), "clear launch");
+            d->planes_dirty = false;
+        }
         stereo::NccParams np{};
-        np.L = pl;
-        np.R = pr;
+        np.L = view_of(left);
+        np.R = view_of(right);
         np.lstats = d->lstats;
         np.rstats = d->rstats;
         np.stats_pitch = W;
         np.lkey = d->lkey;
-        np.rpart = d->rpart;
+        np.rkey = d->rkey;
         np.W = W;
         np.H = H;
         np.D = d->mp.num_disparities;
         np.bx = d->bx;
         np.by = d->by;
         np.ntx = d->ntx;
+        np.rb = d->rb;
         np.nseg = d->nseg;
         np.seg_len = d->seg_len;
         np.bins = bins;
-        np.bins_nty = bins_nty;
+        np.bins_ntx = (W + stereo::BM_TILE_W - 1) / stereo::BM_TILE_W;
+        d->planes_dirty = true;  // until the merge has run
         HIP_TRY(ctx, stereo::launch_ncc(d->mp.window_w, np, s), "ncc launch");
     } else if (aw) {
         if (d->planes_dirty) {
@@ -595,29 +600,22 @@ static stereo_status matcher_run(stereo_driver* d, stereo_image* disp, bool disp
     if (injected_failure())
         return fail(ctx, STEREO_ERROR_HIP, "%s: injected failure between the matcher and the merge", d->name);
     stereo::BmFinishParams f;
-    f.lkey = d->lkey;
-    f.rpart = d->rpart;
-    if (d->rkey) {
-        f.lplane = d->lkey;
-        f.rplane = d->rkey;
-    }
+    f.lplane = d->lkey;
+    f.rplane = d->rkey;
+    f.nlseg = ncc ? d->nseg : 0;
     f.disp = (disp && !dispid) ? view_of(disp) : null_view();
     f.dispid = (disp && dispid) ? view_of(disp) : null_view();
     f.disp_l = disp_lr ? view_of(disp_lr) : null_view();
     f.disp_r = disp_rl ? view_of(disp_rl) : null_view();
     f.W = W;
     f.H = H;
-    f.D = d->mp.num_disparities;
-    f.ntx = d->ntx;
-    f.nseg = d->nseg;
-    f.seg_len = d->seg_len;
     f.bx = d->bx;
     f.by = d->by;
     f.tol = d->mp.lr_tolerance;
     f.value_base = d->mp.algorithm == STEREO_ALGO_AW1 ? 255 * 3 * d->mp.window_w * d->mp.window_w : 0;
     if (!ncc && !aw) f.cnn = d->finish_cnn;
     HIP_TRY(ctx, stereo::launch_bm_finish(f, s), "finish launch");
-    if (d->rkey) d->planes_dirty = false;
+    d->planes_dirty = false;
     return end(d, s);
 }
 

@@ -154,12 +154,11 @@ struct stereo_driver {
     uint8_t* padR = nullptr;
     size_t pad_pitch = 0;
     size_t pad_elem = 0;
-    // keys: per disparity segment for NCC (lkey, rpart; stereo_matcher_scores reads the
-    // left keys after the frame); one plane each for SAD, census and the adaptive windows
-    // (lkey, rkey), cleared by every frame's merge -- planes_dirty when a frame's merge did
-    // not run after its matcher
+    int rb = 0;  // NCC: image rows per tile
+    // key planes (lkey, rkey), cleared by every frame's merge -- planes_dirty when a frame's
+    // merge did not run after its matcher.  NCC's left keys are a plane per disparity segment and
+    // stay after the frame, for stereo_matcher_scores
     uint32_t* lkey = nullptr;
-    uint32_t* rpart = nullptr;
     uint32_t* rkey = nullptr;
     bool planes_dirty = false;
     // the learned proposal's coarse matcher: its merge also writes the network input
@@ -199,7 +198,6 @@ inline void driver_release(stereo_driver* d)
     if (d->padL) (void)hipFree(d->padL);
     if (d->padR) (void)hipFree(d->padR);
     if (d->lkey) (void)hipFree(d->lkey);
-    if (d->rpart) (void)hipFree(d->rpart);
     if (d->rkey) (void)hipFree(d->rkey);
     if (d->lstats) (void)hipFree(d->lstats);
     if (d->rstats) (void)hipFree(d->rstats);

@@ -32,7 +32,6 @@ hipError_t launch_census_pair(const View& src0, const View& dst0, const View* sr
 
 // ---- fused SAD / census matcher -------------------------------------------------
 enum { BM_COST_SAD = 0, BM_COST_CENSUS = 1 };
-constexpr int BM_NPART = 320;     // right-view partial keys per tile row
 constexpr int BM_PAD_LEFT = 320;  // readable columns left of x = 0 in matcher inputs
 constexpr int BM_PAD_RIGHT = 128; // readable columns right of x = W-1
 constexpr int BM_MAX_SEG = 8;     // disparity segments per tile (one workgroup each)
@@ -60,18 +59,16 @@ struct CnnInputTarget {
 };
 
 struct BmFinishParams {
-    // the NCC and adaptive-window matchers' keys: per disparity segment
-    const uint32_t* lkey;   // nseg*W*H
-    const uint32_t* rpart;  // nseg*ntx*H*BM_NPART
-    // the SAD / census matcher's key planes (lplane != nullptr): read, then cleared
-    uint32_t* lplane = nullptr;  // W*H
+    // the key planes: read, then cleared -- but the NCC matcher's left keys (nlseg segments of
+    // W*H, their maximum is the pixel's key) stay for the scores
+    uint32_t* lplane = nullptr;  // W*H, or nlseg*W*H
     uint32_t* rplane = nullptr;  // W*H
+    int nlseg = 0;
     View disp;     // int16 checked map (optional: ptr == nullptr)
     View disp_l;   // int16 left map (optional)
     View disp_r;   // int16 right map (optional)
     View dispid;   // 4 x uint16 reference pixels (optional)
-    int W, H, D, ntx;
-    int nseg, seg_len;
+    int W, H;
     int bx, by, tol;
     int value_base;  // != 0: the 4 x uint16 output carries value_base - cost (AW1 similarity)
     CnnInputTarget cnn{};  // with the key planes: the network input from the checked map `disp`
@@ -150,20 +147,24 @@ hipError_t launch_crosscheck_ref(const View& out, const View& lr, const View& rl
                                  uint32_t* state, uint32_t* result, hipStream_t s);
 
 // ---- NCC matcher ------------------------------------------------------------------
+// Elements past the last one that a statistics array has to have: the matcher reads the left
+// statistics of whole blocks of 32 pixels.
+constexpr int NCC_STATS_PAD = 64;
+
 struct NccParams {
-    View L, R;             // uint8 grey, padded views like the SAD matcher's inputs
-    const int2* lstats;    // per-pixel (S, float bits of 2^23/sqrt(var) or 0)
-    const int2* rstats;    // per-pixel (S, float bits of 1/sqrt(var) or 0)
+    View L, R;             // uint8 grey images
+    const int2* lstats;    // per-pixel (-sum of I - 128, float bits of 2^23/sqrt(var) or 0)
+    const int2* rstats;    // per-pixel (sum of J - 128, float bits of 1/sqrt(var) or 0)
     int stats_pitch;       // elements per stats row
-    uint32_t* lkey;        // nseg*W*H
-    uint32_t* rpart;       // nseg*ntx*H*BM_NPART
+    uint32_t* lkey;        // nseg*W*H: each segment's left keys (matchable rows and columns)
+    uint32_t* rkey;        // W*H right-key plane, zero at the launch (every tile folds in)
     int W, H, D;
     int bx, by;
-    int ntx, nseg, seg_len;
-    // band search: searched 8-disparity bins per 64 x BM_TILE_H tile ([bins_nty][ntx]);
-    // nullptr for the full range
+    int ntx, rb, nseg, seg_len;  // from ncc_grid
+    // band search: searched 8-disparity bins per BM_TILE_W x BM_TILE_H tile, bins_ntx to a
+    // row; nullptr for the full range
     const uint32_t* bins;
-    int bins_nty;
+    int bins_ntx;
 };
 
 struct NccScoreParams {
@@ -177,11 +178,10 @@ struct NccScoreParams {
 };
 
 bool ncc_supported(int ww, int wh, int D);
-void ncc_grid(int W, int H, int D, int* ntx, int* nty, int* nseg, int* seg_len);
-hipError_t launch_ncc_stats(const View& img, int2* out, int pitch_px, int ww, int wh, float scale, hipStream_t s);
+void ncc_grid(int W, int H, int D, int* ntx, int* rb, int* nseg, int* seg_len);
 // Both images of a pair (one size) in one launch.
 hipError_t launch_ncc_stats_pair(const View& img0, int2* out0, float scale0, const View& img1, int2* out1, float scale1,
-                                 int pitch_px, int ww, int wh, hipStream_t s);
+                                 int pitch_px, int ww, hipStream_t s);
 hipError_t launch_ncc(int ww, const NccParams& p, hipStream_t s);
 hipError_t launch_ncc_score(const NccScoreParams& f, hipStream_t s);
 

@@ -150,8 +150,6 @@ stereo_status stereo_matcher_process_noalloc(stereo_context* ctx, const stereo_m
     HIP_TRY(ctx, stereo::launch_bm(census ? stereo::BM_COST_CENSUS : stereo::BM_COST_SAD, p->window_w, bp, s),
             "matcher launch");
     stereo::BmFinishParams f;
-    f.lkey = nullptr;
-    f.rpart = nullptr;
     f.lplane = lkey;
     f.rplane = rkey;
     f.disp = (disp && !dispid) ? view_of(disp) : null_view();
@@ -160,10 +158,6 @@ stereo_status stereo_matcher_process_noalloc(stereo_context* ctx, const stereo_m
     f.disp_r = disp_rl ? view_of(disp_rl) : null_view();
     f.W = W;
     f.H = H;
-    f.D = D;
-    f.ntx = lay.ntx;
-    f.nseg = lay.nseg;
-    f.seg_len = lay.seg_len;
     f.bx = bx;
     f.by = by;
     f.tol = p->lr_tolerance;

@@ -1,6 +1,8 @@
 """GPU NCC matcher against the FP64 oracle: every winning score within 1e-5 relative
 error, disparity maps agreeing except where FP32 rounding reorders a near tie
 (reported and bounded)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -48,6 +50,42 @@ def test_ncc_small(ctx, win):
 
 def test_ncc_tall_segments(ctx):
     _check(ctx, 333, 130, 128, (7, 7), 32, 0.999)
+
+
+@pytest.mark.parametrize("W,H,D,win", [
+    (65, 33, 8, 11), (64, 32, 8, 5), (127, 35, 24, 7), (128, 37, 32, 9), (129, 34, 40, 11), (161, 33, 64, 11),
+    (255, 34, 256, 5), (300, 35, 248, 11), (385, 33, 256, 9), (641, 40, 200, 7)])
+def test_ncc_tiles(ctx, W, H, D, win):
+    """Blocks of 32 x 32 candidates, tiles of 128 columns and 4 or 2 rows, segments of 64 or more
+    disparities: one column and row more and less, ranges that end inside a block, images narrower
+    than their range."""
+    _check(ctx, W, H, D, (win, win), W + D, 0.99)
+
+
+@pytest.mark.parametrize("off,pitch", [(0, 203), (1, 204), (3, 207)])
+def test_ncc_any_alignment(ctx, off, pitch):
+    """Images at any address and row pitch give the maps of the aligned ones."""
+    W, H, D = 201, 37, 64
+    L, R = cs.synth_pair(5, W, H, 0, 8, D - 1, 8)
+    m = cs.Matcher(ctx, W, H, algorithm=cs.ALGO_NCC, window=(11, 11), num_disp=D, tol=1)
+    want = m.run(L, R, maps=True, scores=True)
+
+    class View:
+        def __init__(self, a):
+            raw = np.zeros(off + H * pitch, np.uint8)
+            for y in range(H):
+                raw[off + y * pitch:off + y * pitch + W] = a[y]
+            self.buf = cs.DeviceBuffer.from_array(ctx, raw)
+            self.img = cs.Image(self.buf.ptr.value + off, pitch, cs.ImageFormat(W, H, cs.PIXEL_LUM_U8))
+            self.ref = ctypes.byref(self.img)
+
+    l, r = View(L), View(R)
+    outs = [cs.DeviceImage(ctx, W, H, cs.PIXEL_LUM_I16) for _ in range(3)]
+    m.process(*outs, l, r)
+    score = cs.DeviceImage(ctx, W, H, cs.PIXEL_LUM_F32)
+    cs._check(cs.lib.stereo_matcher_scores(m.handle, score.ref, l.ref, r.ref, None), ctx)
+    for got, ref in zip([o.download() for o in outs] + [score.download()], want):
+        assert np.array_equal(got, ref, equal_nan=got.dtype == np.float32)
 
 
 def test_ncc_config1_rows(ctx):
