@@ -547,11 +547,14 @@ __global__ __launch_bounds__(256) void init_band_mask_kernel(InitBandArgs ib, Cn
     if (t >= ntiles) return;
     const int tx = t % a.ntx, ty = t / a.ntx;
     const int x0 = tx * BM_TILE_W, y0 = ty * BM_TILE_H;
-    const int nx = min(BM_TILE_W, ib.W - x0), ny = min(BM_TILE_H, ib.H - y0);
+    // the initial map's pixels that the tile's pixels read, each once
+    const int X0 = min(x0 / ib.scale, ib.init.w - 1), X1 = (min(x0 + BM_TILE_W, ib.W) - 1) / ib.scale;
+    const int Y0 = min(y0 / ib.scale, ib.init.h - 1), Y1 = (min(y0 + BM_TILE_H, ib.H) - 1) / ib.scale;
+    const int nx = min(X1, ib.init.w - 1) - X0 + 1, ny = min(Y1, ib.init.h - 1) - Y0 + 1;
     int lo = 1 << 30, hi = -1;
+#pragma unroll 4
     for (int k = lane; k < nx * ny; k += 64) {
-        const int y = y0 + k / nx, x = x0 + k % nx;
-        const int X = min(x / ib.scale, ib.init.w - 1), Y = min(y / ib.scale, ib.init.h - 1);
+        const int Y = Y0 + k / nx, X = X0 + k % nx;
         int d;
         if (ib.ref_format) {
             const int id = row_ptr<const ushort4>(ib.init, Y)[X].x;
