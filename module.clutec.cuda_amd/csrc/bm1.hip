@@ -139,8 +139,10 @@ __global__ __launch_bounds__(256) void bm1_kernel(Bm1Args a)
     const bool rows_fit = Y0 + S::TBY <= H;  // the block's test rows lie in the image
     const bool upd = block_ok && rows_fit;   // the block evaluates disparities
     int disp[RPT], mx[RPT], prev[RPT], prev2[RPT], nxt[RPT], nxt2[RPT], last[RPT];
+    bool cannot[RPT];  // the full range: told apart when the results are written
 #pragma unroll
     for (int k = 0; k < RPT; ++k) {
+        cannot[k] = false;
         disp[k] = 0;
         mx[k] = -32767;
         prev[k] = prev2[k] = nxt[k] = nxt2[k] = last[k] = 0;
@@ -166,7 +168,7 @@ __global__ __launch_bounds__(256) void bm1_kernel(Bm1Args a)
             const float mean2 = (float)s2 / (float)(P * P);
             const float sq = mean * mean;
             const float sd = sqrtf(fabsf(mean2 - sq)) / 255.0f * 100.0f;
-            if (sd < a.grad_thresh) disp[k] = B1_CANNOT;
+            cannot[k] = sd < a.grad_thresh;
         }
         const int maxd = a.ltor ? X0 - a.offset + 1 : W - X0 - a.offset;  // MaxDisparity
         d_start = a.dmin;
@@ -306,6 +308,20 @@ __global__ __launch_bounds__(256) void bm1_kernel(Bm1Args a)
                                      : s + vrow[ix0 + k + P - 1] - vrow[ix0 + k - 1];
                     // branch-free: every state value is a select
                     const int v = (int)(int16_t)s;
+                    if (NB > 1) {
+                        // every result's state moves at every disparity of its block, so no
+                        // condition on the result enters: nine VALU operations, not thirteen
+                        const bool above = v > mx[k];
+                        const bool b1 = disp[k] == d + B1_FIRST - 1, b2 = disp[k] == d + B1_FIRST - 2;
+                        prev2[k] = above ? prev[k] : prev2[k];
+                        prev[k] = above ? last[k] : prev[k];
+                        nxt[k] = (above | b1) ? v : nxt[k];
+                        nxt2[k] = (above | b2) ? v : nxt2[k];
+                        disp[k] = above ? d + B1_FIRST : disp[k];
+                        mx[k] = max(mx[k], v);
+                        last[k] = v;
+                        continue;
+                    }
                     const bool act = upd && disp[k] <= B1_LAST;
                     const bool above = act && v > mx[k];
                     const bool b1 = act && !above && disp[k] + 1 == d + B1_FIRST;
@@ -329,7 +345,7 @@ __global__ __launch_bounds__(256) void bm1_kernel(Bm1Args a)
         const int ix = ix0 + k, iy = rr % 4;
         if (!block_ok || !(X0 + ix + P < W && Y0 + iy + P < H)) continue;
         ushort4 o;
-        const int dv = disp[k];
+        const int dv = NB == 1 ? disp[k] : cannot[k] ? B1_CANNOT : upd ? disp[k] : 0;
         if (dv > B1_LAST || dv == 0) {
             o = make_ushort4((uint16_t)dv, 0, 0, 0);
         } else {

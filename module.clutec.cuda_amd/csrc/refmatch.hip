@@ -32,6 +32,8 @@
 // around an initial map (MatcherUseDisparity) runs one block per wave.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "capi_internal.hpp"
 
 namespace stereo {
@@ -162,6 +164,26 @@ __device__ __forceinline__ void track(Tracker& s, int v, int d, bool upd)
     s.last = act ? v : s.last;
 }
 
+// The same update for a search that starts with no disparity, where a result's state moves at
+// every disparity of its block: whether it does at all is decided when it is written, so no
+// condition on the result enters.  Nine VALU operations against thirteen.
+struct Peak {
+    int disp, mx, prev, prev2, nxt, nxt2, last;
+};
+
+__device__ __forceinline__ void track(Peak& s, int v, int d)
+{
+    const bool above = v > s.mx;
+    const bool b1 = s.disp == d + R_FIRST - 1, b2 = s.disp == d + R_FIRST - 2;
+    s.prev2 = above ? s.prev : s.prev2;
+    s.prev = above ? s.last : s.prev;
+    s.nxt = (above | b1) ? v : s.nxt;
+    s.nxt2 = (above | b2) ? v : s.nxt2;
+    s.disp = above ? d + R_FIRST : s.disp;
+    s.mx = max(s.mx, v);
+    s.last = v;
+}
+
 // ------------------------------------------------------------------------------------
 // NCC
 // ------------------------------------------------------------------------------------
@@ -241,12 +263,13 @@ __global__ __launch_bounds__(64) void ncc_ref_kernel(RefArgs a)
     __syncthreads();
 
     bool written[CG];
-    Tracker tr[CG];
+    using State = typename std::conditional<NB == 1, Tracker, Peak>::type;
+    State tr[CG];
     float bmean[CG], bsd[CG];
 #pragma unroll
     for (int k = 0; k < CG; ++k) {
         written[k] = block_ok && X0 + ix0 + k + P < W && Y0 + iy + P < H;
-        tr[k] = Tracker{0, 0, 0, 0, 0, 0, 0};
+        tr[k] = State{};
     }
 
     // left window sums (EvalMsd) and, for the matcher, the gradient sums (EvalGrad): the
@@ -332,7 +355,7 @@ __global__ __launch_bounds__(64) void ncc_ref_kernel(RefArgs a)
         bool any = false;
 #pragma unroll
         for (int k = 0; k < CG; ++k) {
-            tr[k].disp = cannot[k] ? R_CANNOT : 0;
+            if (NB == 1) tr[k].disp = cannot[k] ? R_CANNOT : 0;
             any = any || !cannot[k];
         }
         const uint64_t bal = __ballot(any);
@@ -472,7 +495,8 @@ __global__ __launch_bounds__(64) void ncc_ref_kernel(RefArgs a)
                     }
                     ncc = fmaxf(0.0f, ncc);
                     const int u = (int)fminf(255.0f, ncc * 255.0f);
-                    track(tr[k], u, d, upd);
+                    if constexpr (NB == 1) track(tr[k], u, d, upd);
+                    else track(tr[k], u, d);
                 }
             }
         }
@@ -482,9 +506,9 @@ __global__ __launch_bounds__(64) void ncc_ref_kernel(RefArgs a)
 #pragma unroll
     for (int k = 0; k < CG; ++k) {
         if (!written[k]) continue;
-        const Tracker& s = tr[k];
+        const State& s = tr[k];
         ushort4 o;
-        const int dv = s.disp;
+        const int dv = NB == 1 ? s.disp : cannot[k] ? R_CANNOT : upd ? s.disp : 0;
         if (dv > R_LAST || dv == 0) {
             o = make_ushort4((uint16_t)dv, 0, 0, 0);
         } else {
@@ -815,7 +839,8 @@ __global__ __launch_bounds__(256) void aw1_ref_stack_kernel(RefArgs a)
     // this thread's results: positions l + 256 q of the stack's PCX x RROWS, row-major
     int rx[RPT], ry[RPT], rb[RPT];
     bool has[RPT], written[RPT], upd[RPT];
-    Tracker tr[RPT];
+    Peak tr[RPT];
+    bool cannot[RPT];
 #pragma unroll
     for (int q = 0; q < RPT; ++q) {
         const int pos = l + 256 * q;
@@ -826,7 +851,8 @@ __global__ __launch_bounds__(256) void aw1_ref_stack_kernel(RefArgs a)
         const bool block_ok = by0 + rb[q] < a.nby && X0 + P3 <= W && yb + P3 <= H;
         has[q] = pos < NRES && block_ok;
         written[q] = has[q] && X0 + rx[q] + P3 < W && Y0 + ry[q] + P3 < H;
-        tr[q] = Tracker{0, -32767, 0, 0, 0, 0, 0};
+        tr[q] = Peak{0, -32767, 0, 0, 0, 0, 0};
+        cannot[q] = false;
     }
     __syncthreads();
 
@@ -865,8 +891,8 @@ __global__ __launch_bounds__(256) void aw1_ref_stack_kernel(RefArgs a)
         const float sq = m * m;
         const int isd = (int)sqrtf(fabsf(m2 - sq));
         const float sd = (float)isd / 255.0f * 100.0f;
-        if (sd < a.grad_thresh) tr[q].disp = R_CANNOT;
-        else sflag[rb[q]] = 1;
+        cannot[q] = sd < a.grad_thresh;
+        if (!cannot[q]) sflag[rb[q]] = 1;
     }
     __syncthreads();
 #pragma unroll
@@ -953,7 +979,7 @@ __global__ __launch_bounds__(256) void aw1_ref_stack_kernel(RefArgs a)
                 m2 = max(m2, min(m1, v));
                 m1 = max(m1, v);
                 const int aw = (int)(int16_t)(m1 + m2 + ssp[y + SP][x + SP]);
-                track(tr[q], aw, d, upd[q]);
+                track(tr[q], aw, d);
             }
         }
     }
@@ -962,9 +988,9 @@ __global__ __launch_bounds__(256) void aw1_ref_stack_kernel(RefArgs a)
 #pragma unroll
     for (int q = 0; q < RPT; ++q) {
         if (!written[q]) continue;
-        const Tracker& t = tr[q];
+        const Peak& t = tr[q];
         ushort4 o;
-        const int dv = t.disp;
+        const int dv = cannot[q] ? R_CANNOT : upd[q] ? t.disp : 0;
         if (dv > R_LAST || dv == 0) {
             o = make_ushort4((uint16_t)dv, 0, 0, 0);
         } else {
