@@ -286,19 +286,27 @@ __device__ __forceinline__ void run_job(const Job& j, uint32_t (*hbuf)[HROWS * H
         bm_tile<Cost, AX, AY, false, ATOM>(j, hbuf, ebuf, tid);
 }
 
-// Grid launch over one frame: one workgroup per (tile x, tile y, disparity segment),
-// renumbered so that every XCD works on a contiguous band of tiles.
+// Grid launch over one frame: one workgroup per (tile, disparity segment).  Workgroup b runs on
+// XCD b % 8, which works through an eighth of the tiles in order, a tile's segments together: its
+// segments' atomics meet on the same key-plane lines in one L2, as do the census rows that it and
+// its neighbours read.  The last `tail` tiles of each eighth are cut finer (BmParams).
 template <class Cost, int AX, int AY>
 __global__ __launch_bounds__(256, 2) void bm_fused_kernel(BmParams p)
 {
     __shared__ uint32_t hbuf[2][HROWS * HSTRIDE];
     __shared__ uint32_t ebuf[4][RG][64];
-    // one-dimensional grid of ntx * nty * nseg workgroups
-    const int w = xcd_remap(blockIdx.x, gridDim.x);
-    // segment fastest: the segments of a tile run together on one XCD, so their atomics
-    // on the same key-plane lines meet in its L2, as do the census rows they read
-    const int seg = w % p.nseg, rest = w / p.nseg;
-    const int tx = rest % p.ntx, ty = rest / p.ntx;
+    const int nty = (p.H + TH - 1) / TH, tiles = p.ntx * nty;
+    const int per = (tiles + 7) >> 3;  // tiles of an XCD
+    int i = blockIdx.x >> 3, t = i / p.nseg, seg = i - t * p.nseg, len = p.seg_len;
+    if (t >= per - p.tail) {
+        i -= (per - p.tail) * p.nseg;
+        t = per - p.tail + i / p.tail_nseg;
+        seg = i % p.tail_nseg;
+        len = p.tail_len;
+    }
+    t += (blockIdx.x & 7) * per;
+    if (t >= tiles) return;
+    const int tx = t % p.ntx, ty = t / p.ntx;
     Job j;
     j.L = p.L;
     j.R = p.R;
@@ -307,8 +315,8 @@ __global__ __launch_bounds__(256, 2) void bm_fused_kernel(BmParams p)
     j.bx = p.bx;
     j.x0 = tx * TW;
     j.y0 = ty * TH;
-    j.ds = seg * p.seg_len;
-    j.de = min(p.D, j.ds + p.seg_len);
+    j.ds = seg * len;
+    j.de = min(p.D, j.ds + len);
     // the key planes: every segment of the tile folds into the same rows
     j.rp = p.rkey + (size_t)j.y0 * p.W;
     j.rp_stride = p.W;
@@ -558,9 +566,21 @@ void bm_grid(int W, int H, int D, int* ntx, int* nty, int* nseg, int* seg_len)
 }
 
 template <class Cost>
-static hipError_t launch_cost(const BmParams& p, int ww, hipStream_t s)
+static hipError_t launch_cost(BmParams p, int ww, hipStream_t s)
 {
-    dim3 grid(p.ntx * ((p.H + bm::TH - 1) / bm::TH) * p.nseg);
+    const int per = (p.ntx * ((p.H + bm::TH - 1) / bm::TH) + 7) / 8;
+    p.tail = 0;
+    p.tail_len = p.seg_len;
+    if (p.seg_len == 64) {
+        // The last round of workgroups ends when its longest does, with CUs standing idle: the last
+        // quarter of an XCD's tiles, or about the round that its 32 CUs hold, goes in half as long
+        // segments (1920x1080 D=256: frame 255.7 -> 247.3 us; all of it so: 255.7, since a segment
+        // costs its set-up and its atomics; quarter-length ones: 252.0)
+        p.tail = per / 4 < 18 ? per / 4 : 18;
+        p.tail_len = 32;
+    }
+    p.tail_nseg = (p.D + p.tail_len - 1) / p.tail_len;
+    dim3 grid(8 * ((per - p.tail) * p.nseg + p.tail * p.tail_nseg));
     if (ww == 9) hipLaunchKernelGGL((bm::bm_fused_kernel<Cost, 4, 4>), grid, dim3(256), 0, s, p);
     else if (ww == 7) hipLaunchKernelGGL((bm::bm_fused_kernel<Cost, 3, 3>), grid, dim3(256), 0, s, p);
     else hipLaunchKernelGGL((bm::bm_fused_kernel<Cost, 2, 2>), grid, dim3(256), 0, s, p);

@@ -44,6 +44,9 @@ struct BmParams {
     int W, H, D;
     int bx, by;        // matchable border
     int ntx, nseg, seg_len;
+    // set by the launch: the last `tail` tiles of each XCD's share are cut into tail_nseg
+    // segments of tail_len disparities
+    int tail, tail_nseg, tail_len;
 };
 
 // The learned proposal's network input, written by the merge of the coarse census
