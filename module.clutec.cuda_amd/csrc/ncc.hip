@@ -21,17 +21,17 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "window_mm.hpp"
 
 namespace stereo {
 namespace ncc {
+
+using namespace winmm;
 
 constexpr int XT = 128;       // left pixels of a workgroup's tile: 32 per wave
 constexpr int RBMAX = 4;      // image rows of a tile
 constexpr int RCOLS = XT + 256;  // right pixels x0 - 256 .. x0 + 127 that the tile's candidates reach
 constexpr int MAXROWS = RBMAX + 11;
-
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
 
 // Per-pixel window statistics: .x = centre times the window sum of I - 128 (int; centre -1 for
 // the left image, 1 for the right one, so that a product of the two is -SI SJ), .y = float bits of the
@@ -136,88 +136,6 @@ __global__ __launch_bounds__(256) void ncc_stats_kernel(View img0, int2* out0, f
         }
         sv -= old.x;
         ssv -= old.y;
-    }
-}
-
-// Stages I - 128 of `rows` rows from y0 and dword columns [c0, c1) from x0 (clamped to the image;
-// whole dwords are loaded, at any alignment, where none is cut) in rows of DW dwords.  1 << LOG
-// threads take a row.  COPIES == 4: copy c, CS dwords on, holds the rows shifted by c bytes, so that
-// the bytes from any column on start at a dword of copy (column & 3); with CS 8 mod 32 the 32
-// lanes of a block (8 dwords of each copy) read 32 different banks.
-template <int LOG, int DW, int COPIES, int CS>
-__device__ __forceinline__ void stage_image(uint32_t* dst, const View& img, int x0, int y0, int rows, int c0, int c1)
-{
-    const int c = c0 + (threadIdx.x & ((1 << LOG) - 1)), x = x0 + 4 * c;
-    const bool mine = c < c1;
-    if (mine) {
-        // a column is cut at the image's edge, or whole in all rows
-        const bool whole = x >= 0 && x + 4 <= img.w;
-        int xs[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) xs[j] = clampi(x + j, 0, img.w - 1);
-#pragma unroll 5
-        for (int r = threadIdx.x >> LOG; r < rows; r += 256 >> LOG) {
-            const uint8_t* row = row_ptr<const uint8_t>(img, clampi(y0 + r, 0, img.h - 1));
-            uint32_t w = 0;
-            if (whole) __builtin_memcpy(&w, row + x, 4);
-            else w = row[xs[0]] | (uint32_t)row[xs[1]] << 8 | (uint32_t)row[xs[2]] << 16 | (uint32_t)row[xs[3]] << 24;
-            dst[r * DW + c] = w ^ 0x80808080u;
-        }
-    }
-    if (COPIES == 1) return;
-    __syncthreads();
-    if (mine) {
-        for (int r = threadIdx.x >> LOG; r < rows; r += 256 >> LOG) {
-            // (the last column takes a neighbour that no window reaches)
-            const uint32_t* q = dst + r * DW + c;
-            const uint32_t lo = q[0], hi = q[1];
-#pragma unroll
-            for (int k = 1; k < COPIES; ++k) dst[k * CS + r * DW + c] = __builtin_amdgcn_alignbyte(hi, lo, k);
-        }
-    }
-}
-
-// How a P x P window lies in the K of v_mfma_i32_32x32x32_i8.  A window row is DWR dwords (the bytes
-// past its P are zero in the left operand, so the right one may hold anything there); the first
-// HR rows are the operand of lanes 0 .. 31, the rest that of lanes 32 .. 63, each a run of dwords
-// cut into steps of four.
-template <int P>
-struct Shape {
-    static constexpr int DWR = (P + 3) / 4;
-    static constexpr int HR = (P + 1) / 2;
-    static constexpr int STEPS = (HR * DWR + 3) / 4;
-    static constexpr int ROWS = 2 * HR;  // image rows an operand reads (the last one zero in the left)
-    static constexpr uint32_t TAIL = P % 4 == 1 ? 0xFFu : 0xFFFFFFu;  // window bytes of a row's last dword
-};
-
-// The K bytes of one lane's window, the first two dwords of each of its half's rows, then the third
-// ones: a pair is one read that lands as it lies in the operand.  src: the dword that holds the
-// lane's first column, in its half's first row, rows DW dwords apart.  LEFT: of the single copy,
-// shifted here by the column's low bits.
-template <int P, int DW, bool LEFT>
-__device__ __forceinline__ void load_operand(v4i (&v)[Shape<P>::STEPS], const uint32_t* src, int half, uint32_t shift)
-{
-    using S = Shape<P>;
-    static_assert(S::DWR == 2 || S::DWR == 3, "window rows of two or three dwords");
-#pragma unroll
-    for (int k = 0; k < 4 * S::STEPS; ++k) {
-        const int t = k - 2 * S::HR;  // >= 0: a third dword, or past the end, where zeros meet
-        const int r = t < 0 ? k / 2 : min(t, S::HR - 1), j = t < 0 ? k % 2 : S::DWR - 1;
-        if (LEFT) {
-            uint32_t d = __builtin_amdgcn_alignbyte(src[r * DW + j + 1], src[r * DW + j], shift);
-            if (j == S::DWR - 1) d &= S::TAIL;
-            if (t >= (S::DWR - 2) * S::HR || (r == S::HR - 1 && half)) d = 0u;  // past the end, row P
-            v[k / 4][k % 4] = (int)d;
-        } else if (t < 0) {
-            if (k % 2 == 0) {
-                uint64_t two;
-                __builtin_memcpy(&two, src + r * DW, 8);
-                v[k / 4][k % 4] = (int)(uint32_t)two;
-                v[k / 4][k % 4 + 1] = (int)(uint32_t)(two >> 32);
-            }
-        } else {
-            v[k / 4][k % 4] = (int)src[r * DW + j];
-        }
     }
 }
 
@@ -398,7 +316,8 @@ __global__ __launch_bounds__(256, 3) void ncc_mm_kernel(NccParams p)
 #pragma unroll
             for (int r = 0; r < 16; ++r) lacc[r] = 0u;
             v4i av[S::STEPS];
-            load_operand<P, LDW, true>(av, lsrc + i * LDW, half, n & 3);
+            load_operand_shifted<P, LDW>(av, lsrc + i * LDW, n & 3);
+            mask_row<P>(av, S::HR - 1, half ? 0u : ~0u);  // row P
             // left statistics of rows c_r + 4 half: groups of four pixels (the array has room past W)
             int nsi[16];
             float rfi[16];
@@ -412,7 +331,7 @@ __global__ __launch_bounds__(256, 3) void ncc_mm_kernel(NccParams p)
             const int2* const rs = p.rstats + (size_t)y * p.stats_pitch;
             auto products = [&](int kk) {
                 v4i bv[S::STEPS];
-                load_operand<P, RDW, false>(bv, rsrc + i * RDW - 8 * kk, half, 0u);
+                load_operand<P, RDW>(bv, rsrc + i * RDW - 8 * kk);
                 v16i acc = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
                 for (int s = 0; s < S::STEPS; ++s) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[s], bv[s], acc, 0, 0, 0);

@@ -22,19 +22,23 @@
 // Floating point is evaluated as written: contraction off, correctly rounded division and
 // square root, so the byte scores and 16-bit channels equal the oracle's bit for bit.
 //
-// Layout on gfx950: one wave per workgroup.  NCC: a wave takes two vertically adjacent
-// reference blocks of one block column (they share their groups), and lane 32 b + t plays
-// the reference thread t of block b, holding the same CG results.  Per group of 16
-// disparities the right rows sit in LDS with the right windows' mean and deviation; per
-// disparity each lane forms one column's running 16-row sums of L R into LDS, then
-// its results' running row sums and the score.  AW1: a wave takes one reference block;
-// per disparity the column sums, then the sub-patch sums go through LDS.  The band search
-// around an initial map (MatcherUseDisparity) runs one block per wave.
+// Layout on gfx950.  NCC, full range: without a negative offset every result of a block
+// column sees one run of disparities, so the window sums of products are matrix products
+// (ncc_ref_mm_kernel).  With a negative offset, where cut groups place test patches of their
+// own, and in the band search around an initial map (MatcherUseDisparity): one wave per
+// workgroup, which takes two vertically adjacent reference blocks of one block column (they
+// share their groups; the band search takes one), and lane 32 b + t plays the reference
+// thread t of block b, holding the same CG results.  Per group of 16 disparities the right
+// rows sit in LDS with the right windows' mean and deviation; per disparity each lane forms
+// one column's running 16-row sums of L R into LDS, then its results' running row sums and
+// the score.  AW1: a wave takes one reference block; per disparity the column sums, then the
+// sub-patch sums go through LDS; the band search runs one block per wave too.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
 
 #include "capi_internal.hpp"
+#include "window_mm.hpp"
 
 namespace stereo {
 namespace {
@@ -526,6 +530,262 @@ __global__ __launch_bounds__(64) void ncc_ref_kernel(RefArgs a)
         }
         row_ptr<ushort4>(a.out, Y0 + iy + P / 2)[X0 + ix0 + k + P / 2] = o;
     }
+}
+
+// The full-range search without a negative offset, where every block of a column sees one run of
+// disparities [dmin, dend): its groups then place every test patch at its own disparity.
+//
+// A workgroup takes 128 result columns of two image rows; wave w the 32 from x0 + 32 w.  The window
+// sums of L R of 32 results against 16 test origins, for both rows, are one matrix product
+// (window_mm.hpp): its rows are the origins of row y (the window's first P of P + 1 image rows)
+// and of row y + 1 (the last P), its columns the results.  A lane then holds one result and, in
+// its 16 registers, the sums at 16 consecutive disparities, which it follows in order; lane n
+// starts n disparities apart from its neighbours.  The test pixels and the test windows' mean and
+// deviation are staged in LDS for 256 disparities at a time.
+//
+// The byte score is trunc(min(255, 255 max(0, num / norm))).  num * ((255 / sd) (1 / sd')) lies
+// within 7 roundings of the reference's float value (4 in it, 3 in the reference's own), at most
+// 1.07e-4 at 255, so it decides the byte except within SCORE_EPS of a whole number, where the
+// division decides.
+//
+// What bounds it: 24 VALU operations per candidate, of which the peak update takes nine and the
+// reference's correctly rounded mean of products four.  1280x720, D = 128, 11x11: 156 us left to
+// right and 148 right to left; 436 each with one column's running sums per lane (ncc_ref_kernel),
+// which carries the sums and both squares through LDS.  113 VGPRs hold four waves per SIMD, as
+// many as 34 KB of LDS do; the windows' statistics come from LDS four registers at a time, since
+// held for all 16 they spill.
+constexpr int MM_XT = 128, MM_CHUNK = 16;                    // results of a row, blocks of 16 disparities staged
+constexpr int MM_TC = MM_XT - 32 + 16 * MM_CHUNK;            // test origins of a chunk
+constexpr float SCORE_EPS = 1.2e-4f;
+
+// One result's run of disparities [dmin, dmin + len): groups of 16 from dmin while they start below
+// the range's end, the last one cut where its test area leaves the image.
+__device__ __forceinline__ int ncc_mm_len(const RefArgs& a, int pcx, int x)
+{
+    const int X0 = x / pcx * pcx, W = a.L.w;
+    const int limit = a.ltor ? X0 - a.offset + 1 : W - 32 - X0 - a.offset;
+    const int stop = min(a.dmax, a.ltor ? X0 - a.offset + 1 : W - X0 - a.offset);
+    if (stop <= a.dmin) return 0;
+    const int groups = (stop - 1 - a.dmin) / R_SDC + 1;
+    return max(0, min(groups * R_SDC, limit - a.dmin));
+}
+
+// Sum, sum of squares (of I) and, for GRAD, of |I(x) - I(x + 1)| of a window row, from its dwords of
+// I - 128 at d.
+template <int P, bool GRAD>
+__device__ __forceinline__ void row_sums(const uint32_t (&d)[(P + 3) / 4], int& s1, int& s2, int& sg)
+{
+    constexpr int ND = (P + 3) / 4;
+    int a = 0, b = 0;
+    uint32_t g = 0;
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+        const uint32_t keep = k == ND - 1 ? winmm::Shape<P>::TAIL : ~0u;
+        const uint32_t v = d[k] & keep;
+        a = __builtin_amdgcn_sdot4((int)v, 0x01010101, a, false);
+        b = __builtin_amdgcn_sdot4((int)v, (int)v, b, false);
+        if (GRAD) {
+            // one column on; I and I - 128 differ by the top bit
+            const uint32_t w = __builtin_amdgcn_alignbyte(k + 1 < ND ? d[k + 1] : 0u, d[k], 1);
+            g = __builtin_amdgcn_sad_u8((v ^ 0x80808080u) & keep, (w ^ 0x80808080u) & keep, g);
+        }
+    }
+    s1 = a + 128 * P;                   // sum of I
+    s2 = b + 256 * a + 16384 * P;       // sum of I^2
+    sg = (int)g;
+}
+
+template <int P, bool LTOR>
+__global__ __launch_bounds__(256, 3) void ncc_ref_mm_kernel(RefArgs a, int xmax, int ymax)
+{
+#pragma clang fp contract(off)
+    using namespace winmm;
+    using S = Shape<P>;
+    constexpr int N = P * P, PCX = NccShape<P>::PCX;
+    constexpr int RDW = MM_TC / 4 + 3, LDW = MM_XT / 4 + 3, ND = S::DWR;
+    constexpr int RCS = ((S::ROWS * RDW + 23) & ~31) + 8;
+    static_assert(RCS > S::ROWS * RDW && RCS % 32 == 8, "whole copies, in different banks");
+    __shared__ uint32_t rimg[4 * RCS];
+    __shared__ uint32_t limg[S::ROWS * LDW];
+    // test windows of both rows: mean, deviation, 1 / deviation, 128 sum
+    __shared__ __align__(16) float tmean[2][MM_TC], tsd[2][MM_TC], trsd[2][MM_TC];
+    __shared__ __align__(16) int tsum[2][MM_TC];
+    __shared__ float4 bst[2][MM_XT];   // base windows: mean, deviation, 128 sum - 16384 N, mean gradient
+
+    const int W = a.L.w, H = a.L.h;
+    const int x0 = blockIdx.x * MM_XT, y = 2 * blockIdx.y;
+    const int lane = threadIdx.x & 63, n = lane & 31, half = lane >> 5;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int xb = x0 + 32 * wv, x = xb + n;
+
+    stage_image<6, LDW, 1, 0>(limg, a.L, x0, y, S::ROWS, 0, LDW);
+    __syncthreads();
+    if (threadIdx.x < MM_XT) {
+        const int c = threadIdx.x;
+        int t1 = 0, t2 = 0, tg = 0, e1[2] = {}, e2[2] = {}, eg[2] = {};
+#pragma unroll
+        for (int r = 0; r < S::ROWS; ++r) {
+            const uint32_t* q = limg + r * LDW + (c >> 2);
+            uint32_t d[ND];
+#pragma unroll
+            for (int k = 0; k < ND; ++k) d[k] = __builtin_amdgcn_alignbyte(q[k + 1], q[k], c & 3);
+            int s1, s2, sg;
+            row_sums<P, true>(d, s1, s2, sg);
+            t1 += s1;
+            t2 += s2;
+            tg += sg;
+            if (r == 0) e1[1] = s1, e2[1] = s2, eg[1] = sg;                    // not in row y + 1's window
+            if (r == S::ROWS - 1) e1[0] = s1, e2[0] = s2, eg[0] = sg;          // not in row y's
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int s1 = t1 - e1[h];
+            const float m = div_window<N>(s1), m2 = div_window<N>(t2 - e2[h]), sq = m * m;
+            bst[h][c] = make_float4(m, sqrtf(m2 - sq), __int_as_float(128 * s1 - 16384 * N), div_window<N>(tg - eg[h]));
+        }
+    }
+    __syncthreads();
+
+    const float4 base = bst[half][32 * wv + n];
+    const float bmean = base.x, bsd = base.y, rb = 255.0f / base.y;
+    const int cl = __float_as_int(base.z);
+    const bool cannot = base.w < a.grad_thresh;
+    const bool mine = x < xmax && y + half < ymax;
+    const int len = mine ? ncc_mm_len(a, PCX, x) : 0;
+    // the run grows with x left to right, shrinks right to left: the longest of the wave, of the tile
+    const int xw = LTOR ? min(xb + 31, xmax - 1) : xb, xt = LTOR ? min(x0 + MM_XT, xmax) - 1 : x0;
+    const int lenw = xb < xmax ? ncc_mm_len(a, PCX, xw) : 0, lent = ncc_mm_len(a, PCX, xt);
+    const int nbw = lenw > 0 ? (lenw + 31 + 15) / 16 : 0, nbt = lent > 0 ? (lent + 31 + 15) / 16 : 0;
+
+    v4i bv[S::STEPS];
+    load_operand_shifted<P, LDW>(bv, limg + half * S::HR * LDW + 8 * wv + (n >> 2), n & 3);
+    // the test operand's lane: origin r of image row y + hm; register r of the result is row
+    // 8 (r / 4) + 4 hm + r % 4 of the product
+    const int rm = 4 * (n >> 3) + (n & 3), hm = (n >> 2) & 1;
+    const int at0 = LTOR ? 16 * MM_CHUNK - 1 + 32 * wv - rm : 32 * wv + rm;  // its column of the chunk, block 0
+    const uint32_t* const tsrc = rimg + (at0 & 3) * RCS + half * S::HR * RDW + (at0 >> 2);
+    const uint32_t keep_first = (half == 0 && hm == 1) ? 0u : ~0u, keep_last = (half == 1 && hm == 0) ? 0u : ~0u;
+    // the lane's disparity, less dmin, in register 0 of block 0
+    const int lag0 = LTOR ? n - 31 : -n;
+
+    Peak pk{};
+    for (int c = 0; c < nbt; c += MM_CHUNK) {
+        const int col0 = LTOR ? x0 + 31 - a.offset - a.dmin - 16 * (c + MM_CHUNK) + 1 : x0 + a.offset + a.dmin + 16 * c;
+        __syncthreads();  // the previous chunk has been read
+        stage_image<7, RDW, 4, RCS>(rimg, a.R, col0, y, S::ROWS, 0, RDW);
+        __syncthreads();
+        for (int i = threadIdx.x; i < MM_TC; i += 256) {
+            const uint32_t* q = rimg + (i & 3) * RCS + (i >> 2);
+            int t1 = 0, t2 = 0, e1[2] = {}, e2[2] = {}, unused;
+#pragma unroll
+            for (int r = 0; r < S::ROWS; ++r) {
+                uint32_t d[ND];
+#pragma unroll
+                for (int k = 0; k < ND; ++k) d[k] = q[r * RDW + k];
+                int s1, s2;
+                row_sums<P, false>(d, s1, s2, unused);
+                t1 += s1;
+                t2 += s2;
+                if (r == 0) e1[1] = s1, e2[1] = s2;
+                if (r == S::ROWS - 1) e1[0] = s1, e2[0] = s2;
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int s1 = t1 - e1[h];
+                const float m = div_window<N>(s1), m2 = div_window<N>(t2 - e2[h]), sq = m * m;
+                const float sd = sqrtf(m2 - sq);
+                tmean[h][i] = m;
+                tsd[h][i] = sd;
+                trsd[h][i] = 1.0f / sd;
+                tsum[h][i] = 128 * s1;
+            }
+        }
+        __syncthreads();
+        const int kend = min(c + MM_CHUNK, nbw);
+        for (int k = c; k < kend; ++k) {
+            const int kk = k - c, step = LTOR ? -4 * kk : 4 * kk;
+            v4i av[S::STEPS];
+            load_operand<P, RDW>(av, tsrc + step);
+            mask_row<P>(av, 0, keep_first);
+            mask_row<P>(av, S::HR - 1, keep_last);
+            // the test windows of registers 4 g .. 4 g + 3, of this lane's image row: four columns,
+            // in falling order left to right
+            const int t0 = LTOR ? 16 * MM_CHUNK - 4 + 32 * wv - 16 * kk : 32 * wv + 16 * kk;
+            auto four = [&](const auto* col, int g) { return reinterpret_cast<const float4*>(col + t0 + (LTOR ? -4 * g : 4 * g))[0]; };
+            auto pick = [](const float4& v, int e) {
+                const float f[4] = {v.x, v.y, v.z, v.w};
+                return f[LTOR ? 3 - e : e];
+            };
+            v16i acc;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const float4 v = four(tsum[half], g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[4 * g + e] = __float_as_int(pick(v, e));
+            }
+#pragma unroll
+            for (int s = 0; s < S::STEPS; ++s) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[s], bv[s], acc, 0, 0, 0);
+            const int lag = lag0 + 16 * k;
+            const bool whole = __ballot(lag < 0 || lag + 16 > len) == 0;
+            const int d0 = a.dmin + lag;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const float4 tm = four(tmean[half], g), td = four(tsd[half], g), tr = four(trsd[half], g);
+                int u[4];
+                float num[4], norm[4];
+                bool near = false;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int r = 4 * g + e;
+                    const float cross = div_window<N>(acc[r] + cl);
+                    const float mm = bmean * pick(tm, e);
+                    num[e] = cross - mm;
+                    norm[e] = bsd * pick(td, e);
+                    const float t = __builtin_amdgcn_fmed3f(num[e] * (rb * pick(tr, e)), 0.5f, 255.5f);
+                    near = near | (__builtin_amdgcn_fractf(t + SCORE_EPS) < 2.0f * SCORE_EPS);
+                    u[e] = norm[e] < 1.0f ? 0 : (int)t;
+                }
+                if (__ballot(near)) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float ncc = norm[e] < 1.0f ? 0.0f : num[e] / norm[e];
+                        ncc = fmaxf(0.0f, ncc);
+                        u[e] = (int)fminf(255.0f, ncc * 255.0f);
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int r = 4 * g + e;
+                    if (whole) {
+                        track(pk, u[e], d0 + r);
+                    } else if ((uint32_t)(lag + r) < (uint32_t)len) {
+                        track(pk, u[e], d0 + r);
+                    }
+                }
+            }
+        }
+    }
+
+    // WriteDisparity (:491-592)
+    if (!mine || x + P >= W || y + half + P >= H) return;
+    ushort4 o;
+    const int dv = cannot ? R_CANNOT : pk.disp;
+    if (dv > R_LAST || dv == 0) {
+        o = make_ushort4((uint16_t)dv, 0, 0, 0);
+    } else {
+        const float fmax = (float)pk.mx / 255.0f;
+        const int diff1 = max(abs(pk.prev - pk.mx), abs(pk.prev2 - pk.mx));
+        const int diff2 = max(abs(pk.nxt - pk.mx), abs(pk.nxt2 - pk.mx));
+        int code;
+        if (fmax >= a.sim_thresh) {
+            const bool sat = dv <= R_FIRST + a.dmin + 1 || dv >= R_FIRST + a.dmax - 1;
+            code = sat ? R_SATURATED : ((diff1 >= a.imin_delta && diff2 >= a.imin_delta) ? dv : R_NOT_SPECIFIC);
+        } else {
+            code = R_NOT_FOUND;
+        }
+        o = make_ushort4((uint16_t)code, (uint16_t)pk.mx, (uint16_t)diff1, (uint16_t)diff2);
+    }
+    row_ptr<ushort4>(a.out, y + half + P / 2)[x + P / 2] = o;
 }
 
 // ------------------------------------------------------------------------------------
@@ -1021,9 +1281,15 @@ struct RefExt : DriverExt {
 template <int P>
 hipError_t ncc_ref_launch(const RefArgs& a, int nbx, hipStream_t s)
 {
+    const int xmax = nbx * NccShape<P>::PCX, ymax = a.nby * 16;
     if (a.init.ptr)
         hipLaunchKernelGGL((ncc_ref_kernel<P, 1>), dim3(nbx, a.nby), dim3(64), 0, s, a);
-    else
+    else if (a.offset >= 0) {  // 1280x720, D = 128, 11x11: 156 against 436 us; nothing smaller is slower
+        const dim3 grid((xmax + MM_XT - 1) / MM_XT, ymax / 2);
+        if (a.ltor) hipLaunchKernelGGL((ncc_ref_mm_kernel<P, true>), grid, dim3(256), 0, s, a, xmax, ymax);
+        else hipLaunchKernelGGL((ncc_ref_mm_kernel<P, false>), grid, dim3(256), 0, s, a, xmax, ymax);
+    }
+    else  // a negative offset moves the test patches of cut groups off their disparity
         hipLaunchKernelGGL((ncc_ref_kernel<P, 2>), dim3(nbx, (a.nby + 1) / 2), dim3(64), 0, s, a);
     return hipGetLastError();
 }

@@ -85,6 +85,26 @@ def test_ncc_ref_small_and_ragged(ctx, W, H, patch):
     _check(_ncc(ctx, L, R, **kw), _ncc_oracle(L, R, **kw), f"{W}x{H}")
 
 
+# Edges of the matrix tiles (128 result columns, 2 rows, 16 disparities, 256 staged at a time): one
+# result column of blocks, 127 / 128 / 129 and more results, odd row counts, ranges that begin
+# past 0, end inside a group, span several stagings and reach past the image, and the offsets on
+# either side of the rule that picks the kernel.
+@pytest.mark.parametrize("W,H,patch,ltor,dmin,dmax,off", [
+    (48, 34, 11, True, 0, 64, 0), (139, 40, 11, False, 0, 130, 0), (160, 37, 9, True, 17, 30, 0),
+    (171, 36, 5, False, 3, 100, 4), (700, 31, 11, True, 5, 650, 0), (700, 29, 9, False, 1, 600, 2),
+    (420, 55, 5, True, 250, 300, 1), (331, 30, 11, True, 0, 257, 300), (257, 44, 9, False, 0, 256, 100),
+    (290, 33, 11, True, 0, 70, -1), (290, 33, 5, False, 0, 70, -5),
+])
+def test_ncc_ref_tile_edges(ctx, W, H, patch, ltor, dmin, dmax, off):
+    print(f"ncc_ref tiles {W}x{H} P{patch} ltor{int(ltor)} [{dmin},{dmax}) off {off}", flush=True)
+    L, R = _scene(W + patch, W, H, shifts=(3, 9), ltor=ltor)
+    L[4:22, 10:40] = 90  # no deviation
+    R[2:20, 20:36] = 255
+    kw = dict(patch=patch, disp_min=dmin, disp_max=dmax, disp_offset=off, min_delta_thresh=1, ncc_thresh=0.3,
+              grad_thresh=1.0, left_to_right=ltor)
+    _check(_ncc(ctx, L, R, **kw), _ncc_oracle(L, R, **kw), f"{W}x{H}")
+
+
 @pytest.mark.parametrize("patch,scale", [(11, 2), (9, 4), (5, 1)])
 def test_ncc_ref_band_search_matches_emulation(ctx, patch, scale):
     W, H = 300, 160
