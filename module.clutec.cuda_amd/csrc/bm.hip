@@ -15,12 +15,18 @@
 // are readable memory (values there only meet masked candidates), so the loads
 // need no clamping.  Rows are clamped.
 //
+// What bounds it: VALU issue (221 operations per wave and pair of disparities for census, 17 more
+// for the window's moves) at 2.4 waves per SIMD, with the barrier and the LDS reads behind it.
+//
 // Workgroup = 256 lanes = 4 waves; tile = 64 output columns x 56 output rows; all D
 // disparities are streamed through the tile two at a time:
 //   row phase     lane = (H row 0..63, run of 18 columns).  Costs of the pair
 //                 (d, d+1) are packed as two uint16 halves of one register; the
-//                 right-image window of the lane lives in registers and slides by
-//                 register renaming across 8 disparities.  The horizontal running
+//                 right-image window of the lane lives in registers.  Bytes (SAD): it
+//                 slides by register renaming across 8 disparities, and the next one is
+//                 loaded meanwhile.  64-bit codes (census): 19 of them stay, two come in
+//                 per pair of disparities, loaded a pair ahead, and the window moves up
+//                 every 4 disparities.  The horizontal running
 //                 sum over 2*AX+1 columns takes its halo from the neighbouring runs
 //                 with DPP row shifts, and the sums H go to LDS (double buffered).
 //   column phase  lane = output column, wave = 14-row group.  Vertical running
@@ -49,10 +55,17 @@ constexpr int HSTRIDE = 72;  // == 8 (mod 32): the b64 H stores of a 16-lane gro
 constexpr int RG = TH / 4;
 
 struct CostCensus {
-    static constexpr int DC = 4;  // disparities per right-window load
-    // workgroups per CU asked of the work-list kernel: three fit its LDS, and the
-    // register cap (168) costs it only a few spills outside the disparity loop
-    static constexpr int LIST_WG = 3;
+    static constexpr int DC = 4;  // disparities per turn of the loop
+    // The right window stays in registers: loaded whole for every 4 disparities, 64 lanes of 64
+    // different cache lines each time, it kept the L1 busy for 93 % of the kernel (1920x1080,
+    // D = 256: 129 M accesses, frame 247 us; 44 M and 225 us).  8 disparities a turn, which halve
+    // the moves, need more registers than 168: 228 us.
+    static constexpr bool SLIDE = true;
+    // lane 63 parks what leaves after every disparity; both of a pair at once (as SAD) need
+    // 14 more registers, and the spills cost more than the branch: 226 against 243 us
+    static constexpr bool PAIRS = false;
+    // workgroups per CU: as many as LDS holds, in 168 registers
+    static constexpr int WG = 3;
     using E = uint64_t;           // element type in memory
     struct T { uint32_t lo, hi; };
     static __device__ __forceinline__ T make(E q) { return T{(uint32_t)q, (uint32_t)(q >> 32)}; }
@@ -66,7 +79,11 @@ struct CostCensus {
 
 struct CostSad {
     static constexpr int DC = 8;
-    static constexpr int LIST_WG = 2;  // three would spill inside the disparity loop
+    // the window of 8 disparities is 25 bytes, loaded a turn ahead (20 pairs, 7x7, D up to 256:
+    // 521 -> 507 us)
+    static constexpr bool SLIDE = false;
+    static constexpr bool PAIRS = true;  // 530 -> 521 us there
+    static constexpr int WG = 2;
     using E = uint8_t;
     using T = uint32_t;
     static __device__ __forceinline__ T make(E v) { return v; }
@@ -118,11 +135,18 @@ __device__ __forceinline__ bool job_has_candidates(const Job& j)
 __device__ __forceinline__ uint32_t min_i32(uint32_t a, uint32_t b) { return (int32_t)a < (int32_t)b ? a : b; }
 __device__ __forceinline__ uint32_t plane_key(uint32_t k) { return k ? ~k : 0u; }
 
+// Has v formed here, not later.
+__device__ __forceinline__ void keep14(uint32_t (&v)[14])
+{
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]), "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]), "+v"(v[12]), "+v"(v[13]));
+}
+
 // tid: the thread index (threadIdx.x, or an opaque copy of it, see bm_list_kernel)
 template <class Cost, int AX, int AY, bool EDGE, bool ATOM>
 __device__ __forceinline__ void bm_tile(const Job& p, uint32_t (*hbuf)[HROWS * HSTRIDE], uint32_t (*ebuf)[RG][64],
                                         int tid)
 {
+    constexpr bool SLIDE = Cost::SLIDE;
     static_assert(TH + 2 * AY <= HROWS, "tile too tall for the aggregation window");
     static_assert(AX <= 4, "horizontal radius limited by the run halo");
     constexpr int DC = Cost::DC;
@@ -155,16 +179,35 @@ __device__ __forceinline__ void bm_tile(const Job& p, uint32_t (*hbuf)[HROWS * H
 #pragma unroll
     for (int i = 0; i < RG; ++i) { lacc[i] = 0; racc[i] = 0; }
 
+    typename Cost::T cr[RUN + DC - 1], nx[2];
+    if (SLIDE) {
+#pragma unroll
+        for (int k = DC - 2; k < RUN + DC - 1; ++k) cr[k] = Cost::make(rowR[k]);
+    }
+    uint32_t raw[(RUN + DC + 2) / 4];
+    if (!SLIDE) __builtin_memcpy(raw, rowR, sizeof(raw));
     int s = 0;
     for (int d0 = ds; d0 < de; d0 += DC, rowR -= DC) {
-        typename Cost::T cr[RUN + DC - 1];
+        if (!SLIDE) {
+            // bytes: the window of the next DC disparities is on its way while this one is in use
 #pragma unroll
-        for (int k = 0; k < RUN + DC - 1; ++k) cr[k] = Cost::make(rowR[k]);
+            for (int k = 0; k < RUN + DC - 1; ++k) cr[k] = Cost::make((E)(raw[k >> 2] >> 8 * (k & 3)));
+            __builtin_memcpy(raw, rowR - DC, sizeof(raw));
+        }
 
 #pragma unroll
         for (int q = 0; q < DC / 2; ++q, ++s) {
             const int d = d0 + 2 * q;
             uint32_t* hb = hbuf[s & 1];
+            if (SLIDE) {
+                if (q < DC / 2 - 1) {
+                    cr[DC - 4 - 2 * q] = Cost::make(rowR[DC - 4 - 2 * q]);
+                    cr[DC - 3 - 2 * q] = Cost::make(rowR[DC - 3 - 2 * q]);
+                } else {
+                    nx[0] = Cost::make(rowR[-2]);
+                    nx[1] = Cost::make(rowR[-1]);
+                }
+            }
 
             // ---- row phase: packed costs of (d, d+1) and horizontal sums
             uint32_t e[RUN + 2 * AX];
@@ -209,40 +252,66 @@ __device__ __forceinline__ void bm_tile(const Job& p, uint32_t (*hbuf)[HROWS * H
                 if (EDGE) { k0[i] = ok0 ? k0[i] : 0u; k1[i] = ok1 ? k1[i] : 0u; }
                 lacc[i] = min_i32(lacc[i], min_i32(k0[i], k1[i]));
             }
+            // left to itself the compiler moves these minima below the branches that follow, and
+            // holds all keys of a turn in registers until then (SAD: 194 registers, now 156)
+            keep14(lacc);
             // right-view chain: one lane per step; all rows first so that no DPP read
             // waits on the VALU write just before it, then lane 63 parks what leaves
             static_assert(RG == 14, "the right-view chain block is written for 14 rows");
-            min_shift_in14(racc, k0);
-            if (lane == 63) {
+            if constexpr (Cost::PAIRS) {
+                min_shift_out14(racc, k0);
+                min_shift_out14(k0, k1);
+                if (lane == 63) {
 #pragma unroll
-                for (int i = 0; i < RG; ++i) eb[i * 64 + (d & 63)] = racc[i];
-            }
-            min_shift_in14(racc, k1);
-            if (lane == 63) {
-#pragma unroll
-                for (int i = 0; i < RG; ++i) eb[i * 64 + ((d + 1) & 63)] = racc[i];
-            }
-            // flush the lane-63 emissions every 64 disparities (and at the end)
-            const int dl = d + 1;
-            if ((dl & 63) == 63 || dl == de - 1) {
-                const int base = dl & ~63;
-                if (lane <= (dl & 63) && base + lane >= ds) {
-                    const int k = 318 - (base + lane);
-                    if (ATOM) {
-                        // right pixel x0 + k - 255, inside the image
-                        const int xr = x0 + k - 255;
-                        if (xr >= 0 && xr < W) {
-#pragma unroll
-                            for (int i = 0; i < RG; ++i) {
-                                const uint32_t v = eb[i * 64 + lane];
-                                if (i < rows_here && v) atomicMax(&rp[(size_t)i * p.rp_stride + xr], ~v);
-                            }
-                        }
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < RG; ++i)
-                            if (i < rows_here) rp[i * p.rp_stride + k] = plane_key(eb[i * 64 + lane]);
+                    for (int i = 0; i < RG; ++i) {
+                        const uint32_t both[2] = {k0[i], k1[i]};
+                        __builtin_memcpy(__builtin_assume_aligned(eb + i * 64 + (d & 63), 8), both, 8);
                     }
+                }
+#pragma unroll
+                for (int i = 0; i < RG; ++i) racc[i] = k1[i];
+            } else {
+                min_shift_in14(racc, k0);
+                if (lane == 63) {
+#pragma unroll
+                    for (int i = 0; i < RG; ++i) eb[i * 64 + (d & 63)] = racc[i];
+                }
+                min_shift_in14(racc, k1);
+                if (lane == 63) {
+#pragma unroll
+                    for (int i = 0; i < RG; ++i) eb[i * 64 + ((d + 1) & 63)] = racc[i];
+                }
+            }
+        }
+        if (SLIDE) {
+#pragma unroll
+            for (int k = RUN - 2; k >= 0; --k) cr[k + DC] = cr[k];
+            cr[DC - 2] = nx[0];
+            cr[DC - 1] = nx[1];
+        }
+        // flush the lane-63 emissions every 64 disparities (and at the end)
+        const int dl = d0 + DC - 1;
+        if ((dl & 63) == 63 || dl == de - 1) {
+            // opaque copies: the rows' addresses and bounds are formed here, not held through the loop
+            int stride = p.rp_stride, rows = rows_here, ln = lane;
+            asm volatile("" : "+s"(stride), "+s"(rows), "+v"(ln));
+            const int base = dl & ~63;
+            if (ln <= (dl & 63) && base + ln >= ds) {
+                const int k = 318 - (base + ln);
+                if (ATOM) {
+                    // right pixel x0 + k - 255, inside the image
+                    const int xr = x0 + k - 255;
+                    if (xr >= 0 && xr < W) {
+#pragma unroll
+                        for (int i = 0; i < RG; ++i) {
+                            const uint32_t v = eb[i * 64 + ln];
+                            if (i < rows && v) atomicMax(&rp[(size_t)i * stride + xr], ~v);
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < RG; ++i)
+                        if (i < rows) rp[i * stride + k] = plane_key(eb[i * 64 + ln]);
                 }
             }
         }
@@ -291,10 +360,10 @@ __device__ __forceinline__ void run_job(const Job& j, uint32_t (*hbuf)[HROWS * H
 // segments' atomics meet on the same key-plane lines in one L2, as do the census rows that it and
 // its neighbours read.  The last `tail` tiles of each eighth are cut finer (BmParams).
 template <class Cost, int AX, int AY>
-__global__ __launch_bounds__(256, 2) void bm_fused_kernel(BmParams p)
+__global__ __launch_bounds__(256, Cost::WG) void bm_fused_kernel(BmParams p)
 {
     __shared__ uint32_t hbuf[2][HROWS * HSTRIDE];
-    __shared__ uint32_t ebuf[4][RG][64];
+    __shared__ __align__(8) uint32_t ebuf[4][RG][64];
     const int nty = (p.H + TH - 1) / TH, tiles = p.ntx * nty;
     const int per = (tiles + 7) >> 3;  // tiles of an XCD
     int i = blockIdx.x >> 3, t = i / p.nseg, seg = i - t * p.nseg, len = p.seg_len;
@@ -330,10 +399,10 @@ __global__ __launch_bounds__(256, 2) void bm_fused_kernel(BmParams p)
 // Persistent launch over a work list: each workgroup takes items blockIdx.x,
 // blockIdx.x + gridDim.x, ... up to the device-side count.
 template <class Cost, int AX, int AY>
-__global__ __launch_bounds__(256, Cost::LIST_WG) void bm_list_kernel(BmListParams p)
+__global__ __launch_bounds__(256, Cost::WG) void bm_list_kernel(BmListParams p)
 {
     __shared__ uint32_t hbuf[2][HROWS * HSTRIDE];
-    __shared__ uint32_t ebuf[4][RG][64];
+    __shared__ __align__(8) uint32_t ebuf[4][RG][64];
     __shared__ int next;
     const int n = *p.nitems;
     // Items go out in schedule order: workgroup b takes item b first, with no counter

@@ -124,6 +124,29 @@ __device__ __forceinline__ void min_shift_in14(uint32_t (&acc)[14], const uint32
                  : "v"(key[0]), "v"(key[1]), "v"(key[2]), "v"(key[3]), "v"(key[4]), "v"(key[5]), "v"(key[6]), "v"(key[7]), "v"(key[8]), "v"(key[9]), "v"(key[10]), "v"(key[11]), "v"(key[12]), "v"(key[13]));
 }
 
+// The same with the result in place of the keys: acc holds what it held, so both steps of a pair
+// are there at its end.
+__device__ __forceinline__ void min_shift_out14(const uint32_t (&acc)[14], uint32_t (&key)[14])
+{
+    asm volatile("s_nop 1\n"
+                 "v_min_i32_dpp %0, %14, %0 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 "v_min_i32_dpp %1, %15, %1 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 "v_min_i32_dpp %2, %16, %2 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 "v_min_i32_dpp %3, %17, %3 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 "v_min_i32_dpp %4, %18, %4 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 "v_min_i32_dpp %5, %19, %5 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 "v_min_i32_dpp %6, %20, %6 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 "v_min_i32_dpp %7, %21, %7 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 "v_min_i32_dpp %8, %22, %8 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 "v_min_i32_dpp %9, %23, %9 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 "v_min_i32_dpp %10, %24, %10 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 "v_min_i32_dpp %11, %25, %11 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 "v_min_i32_dpp %12, %26, %12 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 "v_min_i32_dpp %13, %27, %13 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+                 : "+v"(key[0]), "+v"(key[1]), "+v"(key[2]), "+v"(key[3]), "+v"(key[4]), "+v"(key[5]), "+v"(key[6]), "+v"(key[7]), "+v"(key[8]), "+v"(key[9]), "+v"(key[10]), "+v"(key[11]), "+v"(key[12]), "+v"(key[13])
+                 : "v"(acc[0]), "v"(acc[1]), "v"(acc[2]), "v"(acc[3]), "v"(acc[4]), "v"(acc[5]), "v"(acc[6]), "v"(acc[7]), "v"(acc[8]), "v"(acc[9]), "v"(acc[10]), "v"(acc[11]), "v"(acc[12]), "v"(acc[13]));
+}
+
 __device__ __forceinline__ void max_shift_in12(uint32_t (&acc)[12], const uint32_t (&key)[12])
 {
     asm volatile("s_nop 1\n"

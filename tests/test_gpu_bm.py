@@ -80,6 +80,20 @@ def test_matcher_bit_exact(ctx, algo, W, H, D, win, cen):
     assert np.array_equal(out, ref_out)
 
 
+# The right window kept between turns of the disparity loop, and what leaves the tile parked a pair at
+# a time: one turn, an odd number of turns, segments that end inside a block of 64, the last pixel of
+# a tile and the first of the next, and the deepest range, whose last loads reach furthest left.
+@pytest.mark.parametrize("algo", [cs.ALGO_SAD, cs.ALGO_CENSUS])
+@pytest.mark.parametrize("W,H,D", [(64, 56, 8), (65, 57, 24), (127, 113, 72), (129, 30, 104), (321, 61, 248), (577, 40, 256)])
+def test_matcher_window_turns(ctx, algo, W, H, D):
+    print(f"window turns algo={algo} {W}x{H} D={D}", flush=True)
+    cen = (9, 7) if algo == cs.ALGO_CENSUS else (1, 1)
+    L, R = _pair(W + D, W, H, 0, 5, min(D - 1, W // 2))
+    m = cs.Matcher(ctx, W, H, algorithm=algo, window=(7, 7), census=cen, num_disp=D, tol=1)
+    for got, want in zip(m.run(L, R, maps=True), _oracle(algo, L, R, D, (7, 7), cen, 1)):
+        assert np.array_equal(got, want)
+
+
 def test_sad_config0_full(ctx):
     """640x480, D=64, 9x9 SAD, tolerance 1 (the CPU-runnable workload)."""
     L, R = _pair(0, 640, 480, 0, 8, 63)
