@@ -19,6 +19,11 @@
 // the sub-patch sums S at the pixel's column (for rows o-s, o, o+s) and at columns
 // x-s and x+s; the two smallest neighbours come from packed uint16 min/max; the winner
 // key, both winner-take-alls and the right-view chain are those of the SAD matcher.
+//
+// What bounds it: VALU issue and the waits behind the barrier, so it lives on workgroups per
+// CU.  1280x720, D = 128, 5x5 sub-patches, whole frame: 97.7 us with two (rows of 88 words,
+// 212 registers), 82.7 with three, 80.3 with the next window's bytes loaded a turn ahead.
+// The band search needs 182 registers and stays at two.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -30,7 +35,8 @@ constexpr int RG = 12;
 constexpr int TH = 4 * RG;   // 48
 constexpr int HROWS = 64;
 constexpr int RUN = 20;      // 4 runs cover cost columns [-8, 72)
-constexpr int HSTRIDE = 88;
+constexpr int HSTRIDE = 80;  // no padding: the four runs of 20 and the rows fall into different banks, and three
+                             // workgroups fit in LDS
 constexpr int DC = 8;
 
 __device__ __forceinline__ uint32_t pk_min(uint32_t a, uint32_t b)
@@ -43,6 +49,12 @@ __device__ __forceinline__ uint32_t pk_max(uint32_t a, uint32_t b)
 {
     return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned short, a),
                                                                  __builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned short, b)));
+}
+
+// Has v formed here, not later.
+__device__ __forceinline__ void keep12(uint32_t (&v)[12])
+{
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]), "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]));
 }
 
 // BAND: the band search around an initial map (MatcherUseDisparity of BlockMatcherAW1.cu:1336
@@ -106,19 +118,26 @@ __device__ __forceinline__ void aw_tile(const AwParams& p, uint32_t (*hbuf)[HROW
     // the segment) the right-view values parked in the wave's LDS rows go to the partials
     auto flush = [&](int dl) {
         if ((dl & 63) == 63 || dl == de - 1) {
+            // opaque copies: the rows' addresses and bounds are formed here, not held through the loop
+            int stride = W, rows = rows_here, ln = lane;
+            asm volatile("" : "+s"(stride), "+s"(rows), "+v"(ln));
             const int base = dl & ~63;
             // right pixel x0 + 63 - (base + lane), inside the image
-            const int xr = x0 + 63 - (base + lane);
-            if (lane <= (dl & 63) && base + lane >= ds && xr >= 0 && xr < W) {
+            const int xr = x0 + 63 - (base + ln);
+            if (ln <= (dl & 63) && base + ln >= ds && xr >= 0 && xr < W) {
 #pragma unroll
                 for (int i = 0; i < RG; ++i) {
-                    const uint32_t v = eb[i * 64 + lane];
-                    if (i < rows_here && v) atomicMax(&rp[(size_t)i * W + xr], v);
+                    const uint32_t v = eb[i * 64 + ln];
+                    if (i < rows && v) atomicMax(&rp[(size_t)i * stride + xr], v);
                 }
             }
         }
     };
 
+    // the full range: the right bytes of the next DC disparities are on their way while these are
+    // in use
+    uint32_t raw[(RUN + DC + 2) / 4];
+    if (!BAND) __builtin_memcpy(raw, rowR, sizeof(raw));
     int s = 0;
     for (int d0 = ds; d0 < de; d0 += DC, rowR -= DC) {
         // the band search: rows of this wave that search the group (bit o: row o), wave-uniform
@@ -146,8 +165,14 @@ __device__ __forceinline__ void aw_tile(const AwParams& p, uint32_t (*hbuf)[HROW
             }
         }
         uint32_t cr[RUN + DC - 1];
+        if (BAND) {
 #pragma unroll
-        for (int k = 0; k < RUN + DC - 1; ++k) cr[k] = rowR[k];
+            for (int k = 0; k < RUN + DC - 1; ++k) cr[k] = rowR[k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < RUN + DC - 1; ++k) cr[k] = raw[k >> 2] >> 8 * (k & 3) & 255u;
+            __builtin_memcpy(raw, rowR - DC, sizeof(raw));
+        }
 #pragma unroll
         for (int q = 0; q < DC / 2; ++q, ++s) {
             const int d = d0 + 2 * q;
@@ -233,6 +258,9 @@ __device__ __forceinline__ void aw_tile(const AwParams& p, uint32_t (*hbuf)[HROW
                 const uint32_t kk = k0[o] > k1[o] ? k0[o] : k1[o];
                 lacc[o] = lacc[o] > kk ? lacc[o] : kk;
             }
+            // left to itself the compiler moves these maxima below the branches that follow, and
+            // holds all keys of a turn in registers until then
+            keep12(lacc);
             static_assert(RG == 12, "right-view chain written for 12 rows");
             max_shift_in12(racc, k0);
             if (lane == 63) {
@@ -244,8 +272,8 @@ __device__ __forceinline__ void aw_tile(const AwParams& p, uint32_t (*hbuf)[HROW
 #pragma unroll
                 for (int i = 0; i < RG; ++i) eb[i * 64 + ((d + 1) & 63)] = racc[i];
             }
-            flush(d + 1);
         }
+        flush(d0 + DC - 1);
     }
     {
         // what is still in flight belongs to right pixels x0 + lane - (de - 1)
@@ -265,7 +293,7 @@ __device__ __forceinline__ void aw_tile(const AwParams& p, uint32_t (*hbuf)[HROW
 }
 
 template <int SP, bool BAND>
-__global__ __launch_bounds__(256, 2) void aw_fused_kernel(AwParams p)
+__global__ __launch_bounds__(256, BAND ? 2 : 3) void aw_fused_kernel(AwParams p)
 {
     __shared__ uint32_t hbuf[2][HROWS * HSTRIDE];
     __shared__ uint32_t ebuf[4][RG][64];

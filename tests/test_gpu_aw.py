@@ -30,6 +30,18 @@ def test_aw_bit_exact(ctx, algo, mode, W, H, D, sub, kind):
     assert np.array_equal(ids[:, :, 1][v].astype(np.int64), val[v].astype(np.int64))
 
 
+# The loop's turns of 8 disparities with the next window on its way: one turn, several, segments that
+# end inside a block of 64, one column and row past a tile, the deepest range.
+@pytest.mark.parametrize("sub", [3, 5])
+@pytest.mark.parametrize("W,H,D", [(64, 48, 8), (65, 49, 24), (129, 97, 104), (577, 50, 256)])
+def test_aw_window_turns(ctx, W, H, D, sub):
+    print(f"aw turns {W}x{H} D={D} sub={sub}", flush=True)
+    L, R = cs.synth_pair(W + D, W, H, 0, 5, min(D - 1, W // 2), min(8, D - 1))
+    m = cs.Matcher(ctx, W, H, algorithm=cs.ALGO_AW2, window=(sub, sub), num_disp=D, tol=1)
+    for got, want in zip(m.run(L, R, maps=True), orc.aw(2, L, R, D, sub=sub, tol=1, nthreads=8)[:3]):
+        assert np.array_equal(got, want)
+
+
 def test_aw_config2_full(ctx):
     """1280x720 slanted planes, D=128, 15x15 window of 5x5 sub-patches."""
     L, R = cs.synth_pair(2, 1280, 720, 1, 6, 127, 8)
