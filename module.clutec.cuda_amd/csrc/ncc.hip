@@ -151,23 +151,21 @@ __device__ __forceinline__ uint32_t fold_max(uint32_t (&v)[16], int lane)
         const auto sw = __builtin_amdgcn_permlane16_swap(v[r], v[r + 8], false, false);
         a[r] = umax(sw[0], sw[1]);
     }
-#define NCC_DPP(x, ctrl) (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(x), ctrl, 0xf, 0xf, true)
     uint32_t b[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        const uint32_t t0 = umax(a[r], NCC_DPP(a[r], 0x128)), t1 = umax(a[r + 4], NCC_DPP(a[r + 4], 0x128));  // row_ror:8
+        const uint32_t t0 = umax(a[r], dpp_mov<0x128>(a[r])), t1 = umax(a[r + 4], dpp_mov<0x128>(a[r + 4]));  // row_ror:8
         b[r] = (lane & 8) ? t1 : t0;
     }
     uint32_t c[2];
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
-        const uint32_t t0 = umax(b[r], NCC_DPP(b[r], 0x141)), t1 = umax(b[r + 2], NCC_DPP(b[r + 2], 0x141));  // row_half_mirror
+        const uint32_t t0 = umax(b[r], dpp_mov<0x141>(b[r])), t1 = umax(b[r + 2], dpp_mov<0x141>(b[r + 2]));  // row_half_mirror
         c[r] = (lane & 4) ? t1 : t0;
     }
-    const uint32_t t0 = umax(c[0], NCC_DPP(c[0], 0x4E)), t1 = umax(c[1], NCC_DPP(c[1], 0x4E));  // quad_perm [2,3,0,1]
+    const uint32_t t0 = umax(c[0], dpp_mov<0x4E>(c[0])), t1 = umax(c[1], dpp_mov<0x4E>(c[1]));  // quad_perm [2,3,0,1]
     const uint32_t d = (lane & 2) ? t1 : t0;
-    return umax(d, NCC_DPP(d, 0xB1));  // quad_perm [1,0,3,2]
-#undef NCC_DPP
+    return umax(d, dpp_mov<0xB1>(d));  // quad_perm [1,0,3,2]
 }
 
 // Keys of one 32 x 32 block, in the tile's own form: score << 8 | (287 - (xb - x'b) - c_r), the
