@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256) void conv3x3_dw_kernel(CnnDwArgs a)
     uint32_t* const gs = dw_tile + CIN * XS;
     const int lane = threadIdx.x & 63;
     const int col = lane & 15, grp = lane >> 4;
-    const int wv = threadIdx.x >> 6;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     v4f acc[MB][KC][9];
     float bsum[MB];
 #pragma unroll
@@ -256,7 +256,9 @@ __global__ __launch_bounds__(256) void conv3x3_dw_kernel(CnnDwArgs a)
         dw_stage<CIN, XR, 8>(xs, a.x + frame * CIN, a.W, a.H, x0, y0 - DIL);
         dw_stage<COUT, DW_ROWS, 0>(gs, a.dy + frame * COUT, a.W, a.H, x0, y0);
         __syncthreads();
-        for (int kb = 0; kb < 4; ++kb) {
+        // a row past the image has no gradient: its zeros must not meet the rows of X that its taps
+        // lie on, which may hold anything
+        for (int kb = 0; kb < 4 && y0 + wv < a.H; ++kb) {
             const int px = 16 * kb + 4 * grp;  // this lane's four pixels of the row
             v4s av[MB];
 #pragma unroll

@@ -127,6 +127,38 @@ def test_weight_gradient_tiles(ctx, dil, N, H, W):
     assert (np.abs(dwdb[co * 9 * ci:] - rdb) <= tol * mdb).all()
 
 
+@pytest.mark.parametrize("ci,co", [(16, 16), (32, 16), (32, 32)])
+@pytest.mark.parametrize("dil,N,H,W", [(1, 1, 5, 9), (1, 2, 6, 70), (2, 1, 5, 64), (3, 1, 7, 33), (4, 2, 9, 65), (4, 1, 1, 3)])
+def test_weight_gradient_rows_past_the_image(ctx, ci, co, dil, N, H, W):
+    """An infinity in the last row and a NaN in row H - dil (of one channel each) reach the taps that read
+    them and no others: row yy of the gradient meets row yy - dil of X at ky = 0, so these rows meet none
+    there, also where the last tile of 4 rows reaches past the image."""
+    print(f"weight gradient past the image {ci}->{co} dil {dil} {N}x{H}x{W}", flush=True)
+    rng = np.random.default_rng(10 * dil + H + W + ci)
+    x = rng.standard_normal((N, H, W, ci)).astype(np.float32)
+    x[:, H - 1, :, 3] = np.inf
+    x[:, max(H - dil, 0), :, 5] = np.nan
+    xq, xb = _bf16_bits(x)
+    gq, gb = _bf16_bits(rng.standard_normal((N, H, W, co)).astype(np.float32))
+    tx, tg = cs.DeviceBuffer.from_array(ctx, xb), cs.DeviceBuffer.from_array(ctx, gb)
+    tdw = cs.DeviceBuffer(ctx, (co * 9 * ci + co) * 4)
+    cs._check(cs.lib.stereo_conv3x3_bwd_bf16(ctx.handle, tx.ptr, N, H, W, ci, None, tg.ptr, co, dil, None, tdw.ptr, None),
+              ctx)
+    cs._check(cs.lib.stereo_synchronize(ctx.handle, None), ctx)
+    got = tdw.download(np.float32, (co * 9 * ci + co,))
+    w = np.zeros((co, 3, 3, ci), np.float32)
+    with np.errstate(invalid="ignore"):
+        _, rdw, rdb = orc.conv3x3_bwd(xq, w, gq, dil, want_dx=False)
+    fin = np.where(np.isfinite(xq), xq, 0)
+    _, mdw, mdb = orc.conv3x3_bwd(np.abs(fin), w, np.abs(gq), dil, want_dx=False)
+    dw = got[:co * 9 * ci].reshape(co, 3, 3, ci)
+    ok = np.isfinite(rdw)
+    assert ok[:, 0].all() and not ok[:, 1, 1, 3].any() and not ok[:, 1, 1, 5].any()
+    assert np.array_equal(np.isfinite(dw), ok)
+    assert (np.abs(dw[ok] - rdw[ok]) <= 1e-5 * mdw[ok]).all()
+    assert (np.abs(got[co * 9 * ci:] - rdb) <= 1e-5 * mdb).all()
+
+
 def _fill(dc):
     """The coarse-disparity hole filling of the network input (nearest valid to the
     left and right within 64 pixels, the smaller; 0 when none)."""
