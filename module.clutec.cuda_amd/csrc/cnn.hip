@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void conv3x3_kernel(CnnConvArgs a)
 // LDS with the channel outermost, two pixels of a channel in one dword (v_perm_b32 pairs up
 // two 16-byte loads): an operand is then one 8-byte read, and the three horizontal taps of a
 // row come from one 12-pixel run of it by register shifts.  Wave w takes row w of the tile;
-// the waves' sums meet in LDS at the end.
+// the waves' sums meet in LDS at the end (32 -> 32 channels: a block of channels, see the kernel).
 // What bounds it: the two tensors' bytes (33 MB for 16 frames of 240 x 135 at 16 channels) and
 // the LDS transpose; the MFMAs are 2 % of either.  The form it replaces read every operand
 // from global memory two bytes at a time on one wave per workgroup, 2 waves per CU: 163.8 us
@@ -215,19 +215,24 @@ __device__ __forceinline__ void dw_stage(uint32_t* dst, const uint16_t* img, int
     }
 }
 
-// LDS dwords of one workgroup: both staged tiles, and at the end one set of sums
+// LDS dwords of one workgroup: both staged tiles, and at the end one set of sums where waves share it
 template <int CIN, int COUT, int DIL>
 constexpr int dw_lds()
 {
     constexpr int tiles = CIN * dw_stride(DW_ROWS + 2 * DIL, DW_PX) + COUT * dw_stride(DW_ROWS, 64);
-    constexpr int sums = COUT * 9 * CIN + COUT;
+    constexpr int sums = CIN == 32 && COUT == 32 ? 0 : COUT * 9 * CIN + COUT;
     return tiles > sums ? tiles : sums;
 }
 
+// 32 -> 32 channels are four 16 x 16 blocks, one for each wave, which takes all rows of the tile: with
+// the four blocks of a row in one wave (364 registers) the sums of the waves, 36 KB each, were
+// added up one wave after another: stereo_conv3x3_bwd_bf16's call on one tile (9 x 11 pixels, dilation 1)
+// took 38.5 us, now 21.3; on 16 frames of 240 x 135 138 -> 93.
 template <int CIN, int COUT, int DIL>
 __global__ __launch_bounds__(256) void conv3x3_dw_kernel(CnnDwArgs a)
 {
-    constexpr int KC = CIN / 16, MB = COUT / 16;
+    constexpr bool SPLIT = CIN == 32 && COUT == 32;  // a wave takes one block, not one row
+    constexpr int KC = SPLIT ? 1 : CIN / 16, MB = SPLIT ? 1 : COUT / 16;  // blocks of a wave
     constexpr int XR = DW_ROWS + 2 * DIL, XS = dw_stride(XR, DW_PX), GS = dw_stride(DW_ROWS, 64);
     __shared__ __align__(16) uint32_t dw_tile[dw_lds<CIN, COUT, DIL>()];
     uint32_t* const xs = dw_tile;
@@ -235,6 +240,8 @@ __global__ __launch_bounds__(256) void conv3x3_dw_kernel(CnnDwArgs a)
     const int lane = threadIdx.x & 63;
     const int col = lane & 15, grp = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // the wave's first output and input channel
+    const int co0 = SPLIT ? 16 * (wv >> 1) : 0, ci0 = SPLIT ? 16 * (wv & 1) : 0;
     v4f acc[MB][KC][9];
     float bsum[MB];
 #pragma unroll
@@ -258,12 +265,15 @@ __global__ __launch_bounds__(256) void conv3x3_dw_kernel(CnnDwArgs a)
         __syncthreads();
         // a row past the image has no gradient: its zeros must not meet the rows of X that its taps
         // lie on, which may hold anything
-        for (int kb = 0; kb < 4 && y0 + wv < a.H; ++kb) {
-            const int px = 16 * kb + 4 * grp;  // this lane's four pixels of the row
+        const int rows = min(DW_ROWS, a.H - y0);
+        const int nk = SPLIT ? 4 * rows : (wv < rows ? 4 : 0);
+        for (int k = 0; k < nk; ++k) {
+            const int row = SPLIT ? k >> 2 : wv;
+            const int px = 16 * (SPLIT ? k & 3 : k) + 4 * grp;  // this lane's four pixels of the row
             v4s av[MB];
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb) {
-                const uint2 g = *reinterpret_cast<const uint2*>(gs + (mb * 16 + col) * GS + wv * 32 + px / 2);
+                const uint2 g = *reinterpret_cast<const uint2*>(gs + (co0 + mb * 16 + col) * GS + row * 32 + px / 2);
                 av[mb] = __builtin_bit_cast(v4s, g);
                 bsum[mb] += (bf2f(g.x) + bf2f(g.x >> 16)) + (bf2f(g.y) + bf2f(g.y >> 16));
             }
@@ -274,7 +284,7 @@ __global__ __launch_bounds__(256) void conv3x3_dw_kernel(CnnDwArgs a)
             for (int ky = 0; ky < 3; ++ky)
 #pragma unroll
                 for (int kc = 0; kc < KC; ++kc) {
-                    const uint32_t* src = xs + (kc * 16 + col) * XS + (wv + ky * DIL) * (DW_PX / 2) + (px + 4) / 2;
+                    const uint32_t* src = xs + (ci0 + kc * 16 + col) * XS + (row + ky * DIL) * (DW_PX / 2) + (px + 4) / 2;
                     uint32_t v[6];  // pixels px - 4 .. px + 7
 #pragma unroll
                     for (int k = 0; k < 3; ++k) {
@@ -298,38 +308,46 @@ __global__ __launch_bounds__(256) void conv3x3_dw_kernel(CnnDwArgs a)
                 }
         }
     }
-    // the four waves' sums, in wave order, in the layout of the partial sum
     constexpr int NS = COUT * 9 * CIN + COUT;
-    float* const sums = reinterpret_cast<float*>(dw_tile);
+    float* part = a.part + (size_t)blockIdx.x * NS;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
         bsum[mb] += __shfl_xor(bsum[mb], 16);
         bsum[mb] += __shfl_xor(bsum[mb], 32);
     }
-    for (int w = 0; w < 4; ++w) {
-        __syncthreads();
-        if (wv != w) continue;
-        // D[m][n]: lane (col, grp) holds m = 4 grp + i (co), n = col (ci)
+    // D[m][n]: lane (col, grp) holds m = 4 grp + i (co), n = col (ci)
+    if constexpr (SPLIT) {
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
+        for (int t = 0; t < 9; ++t)
 #pragma unroll
-            for (int kc = 0; kc < KC; ++kc)
+            for (int i = 0; i < 4; ++i) part[((co0 + 4 * grp + i) * 9 + t) * CIN + ci0 + col] = acc[0][0][t][i];
+        if (ci0 == 0 && grp == 0) part[COUT * 9 * CIN + co0 + col] = bsum[0];
+    } else {
+        // the four waves' sums, in wave order, in the layout of the partial sum
+        float* const sums = reinterpret_cast<float*>(dw_tile);
+        for (int w = 0; w < 4; ++w) {
+            __syncthreads();
+            if (wv != w) continue;
 #pragma unroll
-                for (int t = 0; t < 9; ++t)
+            for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        float* p = sums + ((mb * 16 + 4 * grp + i) * 9 + t) * CIN + kc * 16 + col;
-                        *p = w ? *p + acc[mb][kc][t][i] : acc[mb][kc][t][i];
-                    }
-            if (grp == 0) {
-                float* p = sums + COUT * 9 * CIN + mb * 16 + col;
-                *p = w ? *p + bsum[mb] : bsum[mb];
+                for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+                    for (int t = 0; t < 9; ++t)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            float* p = sums + ((mb * 16 + 4 * grp + i) * 9 + t) * CIN + kc * 16 + col;
+                            *p = w ? *p + acc[mb][kc][t][i] : acc[mb][kc][t][i];
+                        }
+                if (grp == 0) {
+                    float* p = sums + COUT * 9 * CIN + mb * 16 + col;
+                    *p = w ? *p + bsum[mb] : bsum[mb];
+                }
             }
         }
+        __syncthreads();
+        for (int i = threadIdx.x; i < NS; i += 256) part[i] = sums[i];
     }
-    __syncthreads();
-    float* part = a.part + (size_t)blockIdx.x * NS;
-    for (int i = threadIdx.x; i < NS; i += 256) part[i] = sums[i];
 }
 
 // Adds the partial sums of 16 values per workgroup, 16 threads to a value, in a fixed order.
