@@ -449,7 +449,8 @@ stereo_status stereo_matcher_configure(stereo_context* ctx, stereo_driver** out,
     d->by = p->window_h / 2 + (census ? p->census_h / 2 : 0);
     if (aw) d->bx = d->by = p->window_w + p->window_w / 2;
     if (ncc)
-        stereo::ncc_grid(fmt->width, fmt->height, p->num_disparities, &d->ntx, &d->rb, &d->nseg, &d->seg_len);
+        stereo::ncc_grid(fmt->width, fmt->height, p->num_disparities, p->window_w, p->use_disp_input != 0, &d->ntx, &d->rb,
+                         &d->nseg, &d->seg_len);
     else if (aw)
         stereo::aw_grid(fmt->width, fmt->height, p->num_disparities, &d->ntx, &d->nty, &d->nseg, &d->seg_len);
     else
@@ -462,9 +463,10 @@ stereo_status stereo_matcher_configure(stereo_context* ctx, stereo_driver** out,
     if ((st = driver_events(d))) return cleanup(st);
     if (injected_failure()) return cleanup(fail(ctx, STEREO_ERROR_HIP, "stereo_matcher_configure: injected failure"));
     hipError_t e;
-    // NCC reads the images themselves, and keeps a left key plane per disparity segment
+    // NCC keeps a left key plane per disparity segment, and on the matrix cores reads the images themselves
     const size_t lplanes = ncc ? d->nseg : 1, nstats = W * H + stereo::NCC_STATS_PAD;
-    if (!ncc && ((e = hipMalloc((void**)&d->padL, d->pad_pitch * H)) || (e = hipMalloc((void**)&d->padR, d->pad_pitch * H))))
+    const bool padded = !ncc || d->rb == 0;
+    if (padded && ((e = hipMalloc((void**)&d->padL, d->pad_pitch * H)) || (e = hipMalloc((void**)&d->padR, d->pad_pitch * H))))
         return cleanup(hip_fail(ctx, e, "hipMalloc"));
     // the key planes start at zero; every frame's merge leaves them so
     if ((e = hipMalloc((void**)&d->lkey, lplanes * W * H * 4)) || (e = hipMalloc((void**)&d->rkey, W * H * 4)))
@@ -478,7 +480,8 @@ stereo_status stereo_matcher_configure(stereo_context* ctx, stereo_driver** out,
         if ((e = hipMemset(d->lstats + W * H, 0, stereo::NCC_STATS_PAD * sizeof(int2))) ||
             (e = hipMemset(d->rstats + W * H, 0, stereo::NCC_STATS_PAD * sizeof(int2))))
             return cleanup(hip_fail(ctx, e, "hipMemset"));
-    } else {
+    }
+    if (padded) {
         // the pad columns only ever meet masked candidates; clear them once so that no
         // uninitialised memory is read
         if ((e = hipMemset(d->padL, 0, d->pad_pitch * H)) || (e = hipMemset(d->padR, 0, d->pad_pitch * H)))
@@ -510,12 +513,13 @@ static stereo_status matcher_run(stereo_driver* d, stereo_image* disp, bool disp
     if (census) {
         const View vl = view_of(left), vr = view_of(right);
         HIP_TRY(ctx, stereo::launch_census_pair(vl, pl, &vr, &pr, d->mp.census_w, d->mp.census_h, s), "census launch");
-    } else if (ncc) {
+    } else if (d->padL) {
+        HIP_TRY(ctx, stereo::launch_pad_copy_pair(view_of(left), pl, view_of(right), pr, s), "copy launch");
+    }
+    if (ncc) {
         HIP_TRY(ctx, stereo::launch_ncc_stats_pair(view_of(left), d->lstats, 8388608.0f, view_of(right), d->rstats, 1.0f, W,
                                                    d->mp.window_w, s),
                 "ncc stats launch");
-    } else {
-        HIP_TRY(ctx, stereo::launch_pad_copy_pair(view_of(left), pl, view_of(right), pr, s), "copy launch");
     }
     if (ctx->timing) HIP_TRY(ctx, hipEventRecord(d->ev_stage[0], s), "hipEventRecord");
     if (ncc) {
@@ -525,8 +529,8 @@ static stereo_status matcher_run(stereo_driver* d, stereo_image* disp, bool disp
             d->planes_dirty = false;
         }
         stereo::NccParams np{};
-        np.L = view_of(left);
-        np.R = view_of(right);
+        np.L = d->padL ? pl : view_of(left);
+        np.R = d->padR ? pr : view_of(right);
         np.lstats = d->lstats;
         np.rstats = d->rstats;
         np.stats_pitch = W;

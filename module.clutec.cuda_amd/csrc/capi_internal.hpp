@@ -154,7 +154,7 @@ struct stereo_driver {
     uint8_t* padR = nullptr;
     size_t pad_pitch = 0;
     size_t pad_elem = 0;
-    int rb = 0;  // NCC: image rows per tile
+    int rb = 0;  // NCC: image rows per tile, 0 for the running sums (which read the padded copies)
     // key planes (lkey, rkey), cleared by every frame's merge -- planes_dirty when a frame's
     // merge did not run after its matcher.  NCC's left keys are a plane per disparity segment and
     // stay after the frame, for stereo_matcher_scores

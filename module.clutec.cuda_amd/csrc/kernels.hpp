@@ -155,7 +155,7 @@ hipError_t launch_crosscheck_ref(const View& out, const View& lr, const View& rl
 constexpr int NCC_STATS_PAD = 64;
 
 struct NccParams {
-    View L, R;             // uint8 grey images
+    View L, R;             // uint8 grey images (rb == 0: their padded copies)
     const int2* lstats;    // per-pixel (-sum of I - 128, float bits of 2^23/sqrt(var) or 0)
     const int2* rstats;    // per-pixel (sum of J - 128, float bits of 1/sqrt(var) or 0)
     int stats_pitch;       // elements per stats row
@@ -163,7 +163,7 @@ struct NccParams {
     uint32_t* rkey;        // W*H right-key plane, zero at the launch (every tile folds in)
     int W, H, D;
     int bx, by;
-    int ntx, rb, nseg, seg_len;  // from ncc_grid
+    int ntx, rb, nseg, seg_len;  // from ncc_grid; rb: image rows of a tile, 0 for the running sums
     // band search: searched 8-disparity bins per BM_TILE_W x BM_TILE_H tile, bins_ntx to a
     // row; nullptr for the full range
     const uint32_t* bins;
@@ -181,7 +181,7 @@ struct NccScoreParams {
 };
 
 bool ncc_supported(int ww, int wh, int D);
-void ncc_grid(int W, int H, int D, int* ntx, int* rb, int* nseg, int* seg_len);
+void ncc_grid(int W, int H, int D, int ww, bool band, int* ntx, int* rb, int* nseg, int* seg_len);
 // Both images of a pair (one size) in one launch.
 hipError_t launch_ncc_stats_pair(const View& img0, int2* out0, float scale0, const View& img1, int2* out1, float scale1,
                                  int pitch_px, int ww, hipStream_t s);

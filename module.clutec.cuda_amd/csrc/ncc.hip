@@ -16,7 +16,7 @@
 // of 32 against every right pixel x' of another is one 32 x 32 integer matrix product over the
 // window's N pixels.  Pixels enter as signed bytes I - 128, J - 128: the covariance does not
 // change (SI and SJ shift with them), and every product and sum stays exact in int32.  See
-// ncc_mm_kernel for the layout.
+// ncc_mm_kernel for the layout, and ncc_sums_kernel for short ranges.
 #include <type_traits>
 
 #include "common.hpp"
@@ -394,6 +394,311 @@ __global__ __launch_bounds__(256, 3) void ncc_mm_kernel(NccParams p)
         }
 }
 
+// ------------------------------------------------------------------------------------
+// Short ranges: running sums on the VALU
+// ------------------------------------------------------------------------------------
+// A block of the matrix kernel holds 32 x 32 candidates whatever the range, so a range of 8 costs
+// it as much as one of 32, with the staging and the operands of each row on top.  Running sums
+// cost what the range has, 18.9 VALU operations per candidate.  What bounds them: VALU issue (67 %
+// busy at D = 256) and the barriers behind it.  1920x1080, 11x11, D = 8: frame 54.6 us, 120 with the
+// matrix kernel.  Where the line lies, with both sides measured: ncc_short_range.
+//
+// One disparity per step: workgroup = 4 waves, tile = 64 columns x 52 rows.  Row phase: lane = (H row
+// 0..63, run of 19 columns), products I*J(x-d) and their horizontal sums over 2*AX+1 columns
+// (halo from the neighbouring runs by DPP) into LDS (one buffer, two barriers per disparity).
+// Column phase: lane = column, wave = 13 rows: vertical running sums give SIJ, the right window's
+// (SJ, rJ) come from an LDS tile of the right statistics that is refreshed every 16
+// disparities, the left window's are registers.  Left winner in a register, right winner carried
+// along the wave by a DPP shift (see bm.hip) and folded into the right key plane.  The images
+// are the padded copies (BM_PAD_LEFT), so that the loads need no clamping.
+constexpr int TW = 64;
+constexpr int RG = 13;
+constexpr int TH = 4 * RG;  // 52
+constexpr int HROWS = 64;
+constexpr int RUN = 19;
+constexpr int COLS = 4 * RUN;  // 76 cost columns: tile columns [-6, 70)
+constexpr int HSTRIDE = 76;
+constexpr int DCH = 8;         // disparities per group (one band-search bin)
+constexpr int SDC = 16;        // disparities per right-statistics tile
+constexpr int EMIT = 32;       // right-view values parked per wave between flushes
+constexpr int SCOLS = TW + SDC - 1;
+static_assert(TW == BM_TILE_W, "one column of band-search tiles");
+
+template <int AX, int AY, bool EDGE, bool BAND>
+__device__ __forceinline__ void sums_tile(const NccParams& p, uint32_t* hb, int16_t* ssum, float* srinv,
+                                         uint32_t (*ebuf)[RG][EMIT], int tx, int ty, int seg)
+{
+    static_assert(TH + 2 * AY <= HROWS, "tile too tall for the window");
+    static_assert(AX <= 6 && 2 * AX + 64 <= COLS, "window wider than the run layout");
+    const int tid = threadIdx.x;
+    const int x0 = tx * TW, y0 = ty * TH;
+    const int W = p.W, H = p.H;
+    const int ds = seg * p.seg_len;
+    const int de = min(p.D, ds + p.seg_len);
+    constexpr int N = (2 * AX + 1) * (2 * AY + 1);
+
+    // row phase identity
+    const int run = tid & 3;
+    const int hr = tid >> 2;
+    const int gyr = clampi(y0 - AY + hr, 0, H - 1);
+    const int xs = x0 - 6 + RUN * run;
+    const uint8_t* const rowL = row_ptr<const uint8_t>(p.L, gyr) + xs;
+    const uint8_t* const rowR = row_ptr<const uint8_t>(p.R, gyr) + xs;
+    uint32_t il[RUN];
+#pragma unroll
+    for (int i = 0; i < RUN; ++i) il[i] = rowL[i];
+
+    // column phase identity
+    const int lane = tid & 63;
+    const int gw = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int x = x0 + lane;
+    const int rows_here = H - (y0 + gw * RG);
+    uint32_t* const rp = p.rkey + (size_t)(y0 + gw * RG) * W;
+    uint32_t* const eb = &ebuf[gw][0][0];  // [RG][EMIT]
+    const bool lane_ok = x >= p.bx && x < W - p.bx;
+    const int dlim = x - p.bx;
+    int nsi[RG];     // -SI of the left window
+    float rfi[RG];   // 2^23 / sqrt(varI), or 0
+    uint32_t lacc[RG], racc[RG];
+#pragma unroll
+    for (int i = 0; i < RG; ++i) {
+        const int y = min(y0 + gw * RG + i, H - 1);
+        const int2 st = p.lstats[(size_t)y * p.stats_pitch + min(x, W - 1)];
+        nsi[i] = st.x - 128 * N;
+        rfi[i] = __int_as_float(st.y);
+        lacc[i] = 0;
+        racc[i] = 0;
+    }
+    // band search: the tile's rows lie in at most two 64 x BM_TILE_H bin tiles; rows before
+    // ysplit take m0, the others m1 (uniform per wave and row); a group of disparities
+    // whose bins neither mask holds is skipped
+    uint32_t m0 = ~0u, m1 = ~0u;
+    int ysplit = 1 << 30;
+    if (BAND) {
+        const int tb0 = y0 / BM_TILE_H, tb1 = min(y0 + TH - 1, H - 1) / BM_TILE_H;
+        m0 = p.bins[tb0 * p.bins_ntx + tx];
+        m1 = p.bins[tb1 * p.bins_ntx + tx];
+        ysplit = (tb0 + 1) * BM_TILE_H;
+        const int b0 = ds >> 3, b1 = (de - 1) >> 3;
+        if (((m0 | m1) & (uint32_t)((2ull << b1) - (1ull << b0))) == 0u) {
+            // nothing to search in this segment: every left key is the empty key
+            if (x < W) {
+                uint32_t* lk = p.lkey + (size_t)seg * W * H + (size_t)(y0 + gw * RG) * W + x;
+                for (int i = 0; i < min(RG, rows_here); ++i) lk[(size_t)i * W] = 0u;
+            }
+            return;
+        }
+    }
+
+    // right pixels of the run for the current disparity d, byte i of rw = R(xs + i - d)
+    // (little-endian over RWW words), and the one that enters next, R(xs - d - 1): one load
+    // per disparity instead of RUN (every offset down to xs - de - 1 lies in the matcher's
+    // left padding)
+    constexpr int RWW = (RUN + 3) / 4;
+    // after disparity d: at the end of a block of EMIT disparities (or of the segment) the
+    // right-view values parked in the wave's LDS rows go to the right key plane
+    auto flush = [&](int d) {
+        if ((d & (EMIT - 1)) == EMIT - 1 || d == de - 1) {
+            const int base = d & ~(EMIT - 1);
+            const int xr = x0 + 63 - (base + lane);
+            if (lane <= (d & (EMIT - 1)) && base + lane >= ds && xr >= 0 && xr < W) {
+#pragma unroll
+                for (int i = 0; i < RG; ++i) {
+                    const uint32_t v = eb[i * EMIT + lane];
+                    if (i < rows_here && v) atomicMax(&rp[(size_t)i * W + xr], v);
+                }
+            }
+        }
+    };
+    uint32_t rw[RWW], rnext = 0;
+    int wd = -1;  // the disparity rw holds
+    int sdc = -SDC;  // the first disparity of the right-statistics tile in LDS (none yet)
+    for (int dc = ds; dc < de; dc += DCH) {
+        const int dce = min(de, dc + DCH);
+        // the band search: rows of this wave that search the group (bit r: row r), wave-uniform
+        uint32_t keep = (1u << RG) - 1u;
+        if (BAND) {
+            const uint32_t bit = 1u << (dc >> 3);  // the group's bin (dc is a multiple of 8)
+            const uint32_t lo_rows = (1u << clampi(ysplit - (y0 + gw * RG), 0, RG)) - 1u;
+            keep = ((m0 & bit) ? lo_rows : 0u) | ((m1 & bit) ? (((1u << RG) - 1u) & ~lo_rows) : 0u);
+            if (((m0 | m1) & bit) == 0u) {
+                // no pixel of the tile searches these 8 disparities: the right-view chain
+                // moves on by 8 lanes with no new candidates.  The values that leave the
+                // wave at lane 63 during those 8 steps sit in lanes 62 .. 55 now.
+                if (lane >= 63 - DCH && lane < 63) {
+                    const int slot = (dc + 62 - lane) & (EMIT - 1);
+#pragma unroll
+                    for (int i = 0; i < RG; ++i) eb[i * EMIT + slot] = racc[i];
+                }
+#pragma unroll
+                for (int i = 0; i < RG; ++i) {
+                    const uint32_t v = __shfl_up(racc[i], DCH);
+                    racc[i] = lane >= DCH ? v : 0u;
+                }
+                flush(dce - 1);
+                continue;
+            }
+        }
+        // right statistics for disparities sdc .. sdc+SDC-1 (right columns x0-sdc-(SDC-1) ..
+        // x0+63-sdc), rows of the tile, loaded when the group leaves the tile in LDS: the
+        // thread's loads (the last index repeated past the end) are all issued before the
+        // barrier, the LDS stores after it
+        if (dc - sdc >= SDC) {
+            sdc = dc;
+            constexpr int SN = TH * SCOLS, SIT = (SN + 255) / 256, SB = SIT;
+            static_assert(SIT % SB == 0, "whole batches");
+            // an opaque copy of the thread index: the addresses are recomputed here rather
+            // than hoisted out of the disparity loop into live registers
+            int t0 = tid;
+            asm volatile("" : "+v"(t0));
+            auto sload = [&](int j) {
+                const int k = min(t0 + 256 * j, SN - 1);
+                const int r = k / SCOLS, c = k - r * SCOLS;
+                const int y = min(y0 + r, H - 1);
+                const int xc = clampi(x0 - sdc - (SDC - 1) + c, 0, W - 1);
+                return p.rstats[(size_t)y * p.stats_pitch + xc];
+            };
+#pragma unroll
+            for (int j0 = 0; j0 < SIT; j0 += SB) {
+                int2 v[SB];
+#pragma unroll
+                for (int j = 0; j < SB; ++j) v[j] = sload(j0 + j);
+                if (j0 == 0) __syncthreads();
+#pragma unroll
+                for (int j = 0; j < SB; ++j) {
+                    const int k = tid + 256 * (j0 + j);
+                    if (k < SN) {
+                        ssum[k] = (int16_t)(v[j].x + 128 * N);
+                        srinv[k] = __int_as_float(v[j].y);
+                    }
+                }
+            }
+        }
+        if (wd != dc) {
+            uint32_t b[RUN];
+#pragma unroll
+            for (int i = 0; i < RUN; ++i) b[i] = rowR[i - dc];
+            rnext = rowR[-dc - 1];
+#pragma unroll
+            for (int k = 0; k < RWW; ++k) {
+                uint32_t w = 0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (4 * k + j < RUN) w |= b[4 * k + j] << (8 * j);
+                rw[k] = w;
+            }
+        }
+        for (int d = dc; d < dce; ++d) {
+            // ---- row phase: products and horizontal sums for disparity d
+            uint32_t e[RUN + 2 * AX];
+#pragma unroll
+            for (int i = 0; i < RUN; ++i) e[AX + i] = il[i] * ((rw[i >> 2] >> (8 * (i & 3))) & 0xffu);
+#pragma unroll
+            for (int k = RWW - 1; k > 0; --k) rw[k] = __builtin_amdgcn_alignbyte(rw[k], rw[k - 1], 3);
+            rw[0] = (rw[0] << 8) | rnext;
+            rnext = rowR[-d - 2];
+            wd = d + 1;
+            __syncthreads();  // the previous column phase has read the H buffer
+#pragma unroll
+            for (int i = 0; i < AX; ++i) {
+                e[i] = dpp_mov<DPP_ROW_SHR1>(e[AX + RUN - AX + i]);
+                e[AX + RUN + i] = dpp_mov<DPP_ROW_SHL1>(e[AX + i]);
+            }
+            uint32_t h = 0;
+#pragma unroll
+            for (int i = 0; i <= 2 * AX; ++i) h += e[i];
+            uint32_t* hrow = hb + hr * HSTRIDE + RUN * run;
+#pragma unroll
+            for (int i = 0; i < RUN; ++i) {
+                if (i > 0) h = slide(h, e[i - 1], e[i + 2 * AX]);
+                hrow[i] = h;
+            }
+            __syncthreads();
+
+            // ---- column phase
+            uint32_t hv[RG + 2 * AY];
+            const uint32_t* hcol = hb + gw * RG * HSTRIDE + lane + 6;
+#pragma unroll
+            for (int i = 0; i < RG + 2 * AY; ++i) hv[i] = hcol[i * HSTRIDE];
+            uint32_t sij = 0;
+#pragma unroll
+            for (int i = 0; i <= 2 * AY; ++i) sij += hv[i];
+            const int soff = (gw * RG) * SCOLS + lane + (SDC - 1) - (d - sdc);
+            const int16_t* srow_s = ssum + soff;
+            const float* srow_r = srinv + soff;
+            const uint32_t dd = 255u - (uint32_t)d;
+            bool ok = true;
+            if (EDGE) ok = lane_ok && d <= dlim;
+            uint32_t key[RG];
+#pragma unroll
+            for (int i = 0; i < RG; ++i) {
+                if (i > 0) sij = slide(sij, hv[i - 1], hv[i + 2 * AY]);
+                const int sj = srow_s[i * SCOLS];
+                const int cov = __mul24(nsi[i], sj) + (int)__umul24((uint32_t)N, sij);
+                const float sc = (float)cov * rfi[i] * srow_r[i * SCOLS];
+                // v_cvt_u32_f32 truncates and clamps negative values to 0: the key's
+                // floor(max(score, 0) * 2^23) in one instruction
+                uint32_t q;
+                asm("v_cvt_u32_f32 %0, %1" : "=v"(q) : "v"(sc));
+                uint32_t k = (q << 8) | dd;
+                if (EDGE) k = ok ? k : 0u;
+                if (BAND) k = ((keep >> i) & 1u) ? k : 0u;
+                key[i] = k;
+                lacc[i] = lacc[i] > k ? lacc[i] : k;
+            }
+            static_assert(RG == 13, "right-view chain written for 13 rows");
+            max_shift_in13(racc, key);
+            if (lane == 63) {
+#pragma unroll
+                for (int i = 0; i < RG; ++i) eb[i * EMIT + (d & (EMIT - 1))] = racc[i];
+            }
+            flush(d);
+        }
+    }
+    {
+        // what is still in flight belongs to right pixels x0 + lane - (de - 1)
+        const int xr = x0 + lane - (de - 1);
+        if (xr >= 0 && xr < W) {
+#pragma unroll
+            for (int i = 0; i < RG; ++i)
+                if (i < rows_here && racc[i]) atomicMax(&rp[(size_t)i * W + xr], racc[i]);
+        }
+    }
+    if (x < W) {
+        uint32_t* lk = p.lkey + (size_t)seg * W * H + (size_t)(y0 + gw * RG) * W + x;
+#pragma unroll
+        for (int i = 0; i < RG; ++i)
+            if (i < rows_here) lk[(size_t)i * W] = lacc[i];
+    }
+}
+
+// BAND: the band search's instantiation, a kernel of its own so that the full-range
+// kernel keeps its register count (and three workgroups per CU)
+template <int AX, int AY, bool BAND>
+__global__ __launch_bounds__(256, 3) void ncc_sums_kernel(NccParams p)
+{
+    __shared__ uint32_t hbuf[HROWS * HSTRIDE];
+    // right statistics of the tile: window sums (at most 121 x 255, an int16) and 1/sigma
+    __shared__ int16_t ssum[TH * SCOLS];
+    __shared__ float srinv[TH * SCOLS];
+    __shared__ uint32_t ebuf[4][RG][EMIT];
+    // one-dimensional grid of ntx * nty * nseg workgroups, renumbered per XCD
+    const int nty = (p.H + TH - 1) / TH;
+    // the band search keeps the hardware's round-robin over the XCDs: its work sits in a
+    // few segments and image regions, and a contiguous range per XCD would load some
+    // XCDs far more than others
+    const int w = BAND ? (int)blockIdx.x : xcd_remap(blockIdx.x, gridDim.x);
+    const int tx = w % p.ntx, rest = w / p.ntx;
+    const int ty = rest % nty, seg = rest / nty;
+    const int x0 = tx * TW;
+    const int de = min(p.D, (seg + 1) * p.seg_len);
+    const bool edge = (x0 < p.bx + de - 1) || (x0 + TW > p.W - p.bx);
+    if (edge)
+        sums_tile<AX, AY, true, BAND>(p, hbuf, ssum, srinv, ebuf, tx, ty, seg);
+    else
+        sums_tile<AX, AY, false, BAND>(p, hbuf, ssum, srinv, ebuf, tx, ty, seg);
+}
+
 // Winning score of every left pixel: the same FP32 arithmetic as the matcher, on a
 // window sum computed directly for the winning disparity.
 __global__ __launch_bounds__(256) void ncc_score_kernel(NccScoreParams f)
@@ -435,8 +740,40 @@ bool ncc_supported(int ww, int wh, int D)
     return (ww == 11 && wh == 11) || (ww == 9 && wh == 9) || (ww == 5 && wh == 5) || (ww == 7 && wh == 7);
 }
 
-void ncc_grid(int W, int H, int D, int* ntx, int* rb, int* nseg, int* seg_len)
+// Which kernel a frame takes: the running sums where the range is short and the frame large enough
+// that their two barriers a disparity are hidden (rb = 0).  The matrix kernel costs the same for all
+// ranges up to 32, and more with the window; the running sums hardly see the window.  Whole frames in
+// us, matrix kernel / running sums:
+//                    5x5: D=8      16        24        32        48        64     11x11: 8    16         32         48         64
+//     640 x 480   29.6/29.8  29.8/37.9  29.9/46.8  29.6/42.0  32.3/46.2  31.5/48.7  34.7/29.9  35.1/37.7  34.6/41.9  38.3/47.4  37.0/49.4
+//    1280 x 720   57.6/41.4  57.8/50.9  57.9/61.9  57.2/59.6  66.4/75.9  62.7/83.3  68.7/41.9  69.6/51.8  68.8/60.4  79.1/75.2  75.6/83.7
+//    1920 x 1080  96.2/53.4  96.3/64.8  96.1/79.3  96.0/90.7   114/131    105/132    120/55     120/67     120/92    142/134    132/135
+//    2560 x 1440   158/82     158/100    157/121    156/137    190/209    173/211    198/82     198/101    197/138   235/212    218/214
+// With an initial map the running sums skip what is masked more finely: at 1920 x 1080, a quarter of
+// the size, 11x11, D = 64 150/112, 5x5 119/110; at 1280 x 720 85/67 and 70/65; at 640 x 480 42/51.
+static bool ncc_short_range(int W, int H, int D, int ww, bool band)
 {
+    const double px = (double)W * H;
+    const bool wide = ww >= 9;
+    if (band) return D <= (wide ? 64 : 48) && px >= 880e3;
+    return D <= (wide ? 48 : 32) && px * (wide ? 2 : 1) >= 55e3 * D;
+}
+
+void ncc_grid(int W, int H, int D, int ww, bool band, int* ntx, int* rb, int* nseg, int* seg_len)
+{
+    if (ncc_short_range(W, H, D, ww, band)) {
+        *rb = 0;
+        *ntx = (W + ncc::TW - 1) / ncc::TW;
+        const int tiles = *ntx * ((H + ncc::TH - 1) / ncc::TH);
+        int n = (1200 + tiles - 1) / tiles;
+        if (n > D / 16) n = D / 16;
+        if (n > BM_MAX_SEG) n = BM_MAX_SEG;
+        if (n < 1) n = 1;
+        const int len = ((D + n - 1) / n + 15) & ~15;
+        *seg_len = len;
+        *nseg = (D + len - 1) / len;
+        return;
+    }
     // Tiles of 4 rows where they give every CU four workgroups (three are resident); 2 rows stage
     // more pixels for the same work, so a smaller frame first takes those, and only then splits
     // the disparities, which costs a left key plane per segment.
@@ -471,23 +808,31 @@ hipError_t launch_ncc_stats_pair(const View& img0, int2* out0, float scale0, con
     return hipGetLastError();
 }
 
+template <int P>
+static void launch_ncc_p(const NccParams& p, hipStream_t s)
+{
+    if (p.rb == 0) {
+        const dim3 grid(p.ntx * ((p.H + ncc::TH - 1) / ncc::TH) * p.nseg);
+        if (p.bins) hipLaunchKernelGGL((ncc::ncc_sums_kernel<P / 2, P / 2, true>), grid, dim3(256), 0, s, p);
+        else hipLaunchKernelGGL((ncc::ncc_sums_kernel<P / 2, P / 2, false>), grid, dim3(256), 0, s, p);
+    } else {
+        const dim3 grid(p.ntx * ((p.H + p.rb - 1) / p.rb) * p.nseg);
+        if (p.bins) hipLaunchKernelGGL((ncc::ncc_mm_kernel<P, true>), grid, dim3(256), 0, s, p);
+        else hipLaunchKernelGGL((ncc::ncc_mm_kernel<P, false>), grid, dim3(256), 0, s, p);
+    }
+}
+
 hipError_t launch_ncc(int ww, const NccParams& p, hipStream_t s)
 {
-    if (p.rb < 1 || p.rb > ncc::RBMAX || p.nseg < 1 || p.seg_len % 32 || p.D > 256 || !p.rkey) return hipErrorInvalidValue;
-    dim3 grid(p.ntx * ((p.H + p.rb - 1) / p.rb) * p.nseg);
-#define NCC_LAUNCH(P)                                                                          \
-    if (p.bins)                                                                                   \
-        hipLaunchKernelGGL((ncc::ncc_mm_kernel<P, true>), grid, dim3(256), 0, s, p);               \
-    else                                                                                          \
-        hipLaunchKernelGGL((ncc::ncc_mm_kernel<P, false>), grid, dim3(256), 0, s, p);              \
-    break
+    // segments of whole blocks: 32 disparities, or 16 for the running sums
+    if (p.rb < 0 || p.rb > ncc::RBMAX || p.nseg < 1 || p.seg_len % (p.rb ? 32 : 16) || p.D > 256 || !p.rkey)
+        return hipErrorInvalidValue;
     switch (ww) {
-    case 11: NCC_LAUNCH(11);
-    case 9: NCC_LAUNCH(9);
-    case 7: NCC_LAUNCH(7);
-    default: NCC_LAUNCH(5);
+    case 11: launch_ncc_p<11>(p, s); break;
+    case 9: launch_ncc_p<9>(p, s); break;
+    case 7: launch_ncc_p<7>(p, s); break;
+    default: launch_ncc_p<5>(p, s);
     }
-#undef NCC_LAUNCH
     return hipGetLastError();
 }
 

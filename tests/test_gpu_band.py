@@ -77,7 +77,10 @@ def test_band_search_matches_oracle(ctx, algo, window, scale, fmt):
 
 
 @pytest.mark.parametrize("scale,win,fmt,size", [(2, (11, 11), "i16", (400, 250, 128)), (1, (7, 7), "ref", (400, 250, 128)),
-                                               (4, (9, 9), "i16", (400, 250, 128)), (3, (5, 5), "i16", (333, 190, 64))])
+                                               (4, (9, 9), "i16", (400, 250, 128)), (3, (5, 5), "i16", (333, 190, 64)),
+                                               # large frames of short ranges: the running sums
+                                               (4, (11, 11), "i16", (1111, 801, 64)), (2, (5, 5), "i16", (1111, 801, 48)),
+                                               (1, (9, 9), "ref", (1111, 801, 24))])
 def test_ncc_band_search_matches_oracle(ctx, scale, win, fmt, size):
     """NCC around an initial map (MatcherUseDisparity of BlockMatcherNCC): the oracle's NCC
     restricted to the same per-pixel bins, with the NCC matcher's parity rules: the

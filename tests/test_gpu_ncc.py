@@ -2,6 +2,7 @@
 error, disparity maps agreeing except where FP32 rounding reorders a near tie
 (reported and bounded)."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -62,10 +63,41 @@ def test_ncc_tiles(ctx, W, H, D, win):
     _check(ctx, W, H, D, (win, win), W + D, 0.99)
 
 
-@pytest.mark.parametrize("off,pitch", [(0, 203), (1, 204), (3, 207)])
-def test_ncc_any_alignment(ctx, off, pitch):
+@pytest.mark.parametrize("W,H,D,win", [
+    (1001, 449, 8, 5), (1283, 417, 8, 11), (1283, 701, 16, 7), (961, 701, 24, 9), (1153, 767, 32, 11),
+    (2053, 873, 32, 5), (1291, 1030, 40, 11), (1291, 1030, 48, 9)])
+def test_ncc_short_ranges(ctx, W, H, D, win):
+    """Short ranges of large frames, which take the running sums: ragged tiles of 64 x 52, one group of 8
+    disparities, whole and cut statistics tiles of 16, one to three segments."""
+    assert D <= (48 if win >= 9 else 32) and W * H * (2 if win >= 9 else 1) >= 55000 * D  # the rule
+    _check(ctx, W, H, D, (win, win), W + D, 0.99)
+
+
+def test_ncc_short_range_costs_less(ctx):
+    """A 1920 x 1080 frame of 8 disparities takes clearly less than one of 64 (0.41 of it; 0.91 where all ranges
+    took the same kernel)."""
+    W, H = 1920, 1080
+    L, R = cs.synth_pair(3, W, H, 0, 8, 63, 8)
+    l, r = (cs.DeviceImage.from_array(ctx, a, cs.PIXEL_LUM_U8) for a in (L, R))
+    out = cs.DeviceImage(ctx, W, H, cs.PIXEL_LUM_I16)
+    best = {}
+    for D in (64, 8):
+        m = cs.Matcher(ctx, W, H, algorithm=cs.ALGO_NCC, window=(11, 11), num_disp=D, tol=1)
+        for _ in range(8):
+            t = time.perf_counter()
+            for _ in range(40):
+                m.process(out, None, None, l, r)
+            cs._check(cs.lib.stereo_synchronize(ctx.handle, None), ctx)
+            best[D] = min(best.get(D, 1.0), time.perf_counter() - t)
+    print({d: round(v / 40 * 1e6, 1) for d, v in best.items()}, "us", flush=True)
+    assert best[8] < 0.7 * best[64]
+
+
+@pytest.mark.parametrize("W,H,D,off,more", [(201, 37, 64, 0, 2), (201, 37, 64, 1, 3), (201, 37, 64, 3, 6),
+                                            (1025, 431, 16, 1, 3)])
+def test_ncc_any_alignment(ctx, W, H, D, off, more):
     """Images at any address and row pitch give the maps of the aligned ones."""
-    W, H, D = 201, 37, 64
+    pitch = W + more
     L, R = cs.synth_pair(5, W, H, 0, 8, D - 1, 8)
     m = cs.Matcher(ctx, W, H, algorithm=cs.ALGO_NCC, window=(11, 11), num_disp=D, tol=1)
     want = m.run(L, R, maps=True, scores=True)
