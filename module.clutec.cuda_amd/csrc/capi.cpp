@@ -488,6 +488,9 @@ stereo_status stereo_matcher_configure(stereo_context* ctx, stereo_driver** out,
             return cleanup(hip_fail(ctx, e, "hipMemset"));
     }
     if (p->use_disp_input && (st = band_alloc(d))) return cleanup(st);
+    // hipMemset returns before the null stream has done it, and a frame may come on a stream that
+    // does not wait for that one
+    if ((e = hipDeviceSynchronize()) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipDeviceSynchronize"));
     *out = d;
     return STEREO_OK;
 }

@@ -221,6 +221,8 @@ stereo_status stereo_cnn_create(stereo_context* ctx, stereo_cnn** out, int32_t W
         delete c;
         return st;
     }
+    // the fills and the weights are on the null stream; a set_input may come on one that does not wait for it
+    if ((e = hipDeviceSynchronize())) return bail(e);
     *out = c;
     return STEREO_OK;
 }

@@ -85,3 +85,21 @@ def test_batch_planes_across_frames(ctx):
             got = (b.outs[i].download(), b.lrs[i].download(), b.rls[i].download())
             for a, c in zip(got, want[k][i]):
                 assert np.array_equal(a, c), f"frame {f} (set {k}, pair {i})"
+
+
+@pytest.mark.parametrize("make", [
+    lambda ctx: cs.Matcher(ctx, 16384, 4096, algorithm=cs.ALGO_CENSUS, window=(9, 9), num_disp=64),
+    lambda ctx: cs.Matcher(ctx, 16384, 4096, algorithm=cs.ALGO_SAD, window=(9, 9), num_disp=64),
+    lambda ctx: cs.Matcher(ctx, 16384, 4096, algorithm=cs.ALGO_AW1, window=(5, 5), num_disp=64),
+    lambda ctx: cs.Matcher(ctx, 16384, 4096, algorithm=cs.ALGO_NCC, window=(9, 9), num_disp=64),
+    lambda ctx: cs.CrossCheck(ctx, 640, 480), lambda ctx: cs.ProposalNet(ctx, 1024, 1024, max_frames=8),
+], ids=["census", "sad", "aw1", "ncc", "crosscheck", "network"])
+def test_configured_state_is_in_place(ctx, make):
+    """The planes' first zeros (and the network's labels and weights) are written on the null stream. They are
+    there when the configure call returns, since the first frame may come on a stream that does
+    not wait for that one."""
+    cs._check(cs.lib.stereo_synchronize(ctx.handle, None), ctx)
+    made = make(ctx)
+    busy = cs.lib.hipStreamQuery(None)
+    made.close()
+    assert busy == 0
