@@ -25,7 +25,8 @@
 // Layout on gfx950.  NCC, full range: without a negative offset every result of a block
 // column sees one run of disparities, so the window sums of products are matrix products
 // (ncc_ref_mm_kernel).  With a negative offset, where cut groups place test patches of their
-// own, and in the band search around an initial map (MatcherUseDisparity): one wave per
+// own, for one group of 16 disparities of a large frame (see ncc_ref_launch), and in the band
+// search around an initial map (MatcherUseDisparity): one wave per
 // workgroup, which takes two vertically adjacent reference blocks of one block column (they
 // share their groups; the band search takes one), and lane 32 b + t plays the reference
 // thread t of block b, holding the same CG results.  Per group of 16 disparities the right
@@ -549,9 +550,10 @@ __global__ __launch_bounds__(64) void ncc_ref_kernel(RefArgs a)
 // division decides.
 //
 // What bounds it: 24 VALU operations per candidate, of which the peak update takes nine and the
-// reference's correctly rounded mean of products four.  1280x720, D = 128, 11x11: 156 us left to
-// right and 148 right to left; 436 each with one column's running sums per lane (ncc_ref_kernel),
-// which carries the sums and both squares through LDS.  113 VGPRs hold four waves per SIMD, as
+// reference's correctly rounded mean of products four.  1280x720, D = 128, 11x11: a call takes 144 us
+// left to right and 136 right to left (148 and 143 when all test origins of a chunk were staged,
+// whatever the range); 429 and 425 with one column's running sums per lane (ncc_ref_kernel),
+// which carries the sums and both squares through LDS.  127 VGPRs hold four waves per SIMD, as
 // many as 34 KB of LDS do; the windows' statistics come from LDS four registers at a time, since
 // held for all 16 they spill.
 constexpr int MM_XT = 128, MM_CHUNK = 16;                    // results of a row, blocks of 16 disparities staged
@@ -671,10 +673,14 @@ __global__ __launch_bounds__(256, 3) void ncc_ref_mm_kernel(RefArgs a, int xmax,
     Peak pk{};
     for (int c = 0; c < nbt; c += MM_CHUNK) {
         const int col0 = LTOR ? x0 + 31 - a.offset - a.dmin - 16 * (c + MM_CHUNK) + 1 : x0 + a.offset + a.dmin + 16 * c;
+        // the chunk's test origins that its blocks reach: a short range or the last chunk takes few
+        const int nb = min(MM_CHUNK, nbt - c);
+        const int i0 = LTOR ? 16 * (MM_CHUNK - nb) : 0, i1 = LTOR ? MM_TC : MM_XT - 32 + 16 * nb;
         __syncthreads();  // the previous chunk has been read
-        stage_image<7, RDW, 4, RCS>(rimg, a.R, col0, y, S::ROWS, 0, RDW);
+        if (i1 - i0 <= 4 * (64 - 3)) stage_image<6, RDW, 4, RCS>(rimg, a.R, col0, y, S::ROWS, i0 / 4, i1 / 4 + 3);
+        else stage_image<7, RDW, 4, RCS>(rimg, a.R, col0, y, S::ROWS, i0 / 4, i1 / 4 + 3);
         __syncthreads();
-        for (int i = threadIdx.x; i < MM_TC; i += 256) {
+        for (int i = i0 + threadIdx.x; i < i1; i += 256) {
             const uint32_t* q = rimg + (i & 3) * RCS + (i >> 2);
             int t1 = 0, t2 = 0, e1[2] = {}, e2[2] = {}, unused;
 #pragma unroll
@@ -1282,14 +1288,23 @@ template <int P>
 hipError_t ncc_ref_launch(const RefArgs& a, int nbx, hipStream_t s)
 {
     const int xmax = nbx * NccShape<P>::PCX, ymax = a.nby * 16;
+    // The matrix kernel sums up products for at least 48 disparities of each result and stages the rows they
+    // lie on, so a range of one group of 16 is left to the running sums where the frame is large and the
+    // window costs the matrix kernel most (us, matrix kernel / running sums, [0, 16), left to right):
+    //              5x5       9x9       11x11
+    //  1280x720   47 / 69   58 / 66    60 / 63
+    //  1920x1080 101 / 139 127 / 130  129 / 121
+    //  2560x1440 173 / 203 219 / 195  226 / 185
+    // [0, 32): 261 / 353 and 269 / 331 at the largest; 11x11, 1280x720, [0, 128): 131 / 429.
+    const bool one_group = P >= 9 && a.dmax - a.dmin <= R_SDC && (double)xmax * ymax >= 1.5e6;
     if (a.init.ptr)
         hipLaunchKernelGGL((ncc_ref_kernel<P, 1>), dim3(nbx, a.nby), dim3(64), 0, s, a);
-    else if (a.offset >= 0) {  // 1280x720, D = 128, 11x11: 156 against 436 us; nothing smaller is slower
+    else if (a.offset >= 0 && !one_group) {
         const dim3 grid((xmax + MM_XT - 1) / MM_XT, ymax / 2);
         if (a.ltor) hipLaunchKernelGGL((ncc_ref_mm_kernel<P, true>), grid, dim3(256), 0, s, a, xmax, ymax);
         else hipLaunchKernelGGL((ncc_ref_mm_kernel<P, false>), grid, dim3(256), 0, s, a, xmax, ymax);
     }
-    else  // a negative offset moves the test patches of cut groups off their disparity
+    else  // (a negative offset moves the test patches of cut groups off their disparity)
         hipLaunchKernelGGL((ncc_ref_kernel<P, 2>), dim3(nbx, (a.nby + 1) / 2), dim3(64), 0, s, a);
     return hipGetLastError();
 }

@@ -94,6 +94,10 @@ def test_ncc_ref_small_and_ragged(ctx, W, H, patch):
     (171, 36, 5, False, 3, 100, 4), (700, 31, 11, True, 5, 650, 0), (700, 29, 9, False, 1, 600, 2),
     (420, 55, 5, True, 250, 300, 1), (331, 30, 11, True, 0, 257, 300), (257, 44, 9, False, 0, 256, 100),
     (290, 33, 11, True, 0, 70, -1), (290, 33, 5, False, 0, 70, -5),
+    # nine and ten blocks staged, one block in the second staging and its edge
+    (400, 36, 11, True, 0, 98, 0), (400, 36, 11, False, 0, 99, 0), (420, 35, 9, True, 0, 226, 0), (420, 35, 5, False, 0, 227, 0),
+    # a large frame: one group of 16 disparities (the running sums), and one disparity more
+    (1610, 1005, 11, True, 0, 16, 0), (1613, 1001, 9, False, 2, 14, 3), (1613, 1001, 11, False, 0, 17, 0),
 ])
 def test_ncc_ref_tile_edges(ctx, W, H, patch, ltor, dmin, dmax, off):
     print(f"ncc_ref tiles {W}x{H} P{patch} ltor{int(ltor)} [{dmin},{dmax}) off {off}", flush=True)
