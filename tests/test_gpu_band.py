@@ -78,6 +78,8 @@ def test_band_search_matches_oracle(ctx, algo, window, scale, fmt):
 
 @pytest.mark.parametrize("scale,win,fmt,size", [(2, (11, 11), "i16", (400, 250, 128)), (1, (7, 7), "ref", (400, 250, 128)),
                                                (4, (9, 9), "i16", (400, 250, 128)), (3, (5, 5), "i16", (333, 190, 64)),
+                                               # tiles of 4 rows, the last of 1 row
+                                               (4, (9, 9), "i16", (1023, 769, 192)), (2, (11, 11), "ref", (1025, 769, 72)),
                                                # large frames of short ranges: the running sums
                                                (4, (11, 11), "i16", (1111, 801, 64)), (2, (5, 5), "i16", (1111, 801, 48)),
                                                (1, (9, 9), "ref", (1111, 801, 24))])

@@ -94,6 +94,22 @@ def test_matcher_window_turns(ctx, algo, W, H, D):
         assert np.array_equal(got, want)
 
 
+# Segments of 64 disparities, whose last tiles of each XCD's share go in segments of 32: tiles that are no
+# multiple of 8, a range whose last 64 is cut (4 segments and 7: the last one 8 long), whole ones, and
+# one of 96.
+@pytest.mark.parametrize("algo", [cs.ALGO_SAD, cs.ALGO_CENSUS])
+@pytest.mark.parametrize("W,H,D", [(1283, 901, 200), (1283, 901, 256), (1537, 1345, 96)])
+def test_matcher_tail_segments(ctx, algo, W, H, D):
+    print(f"tail segments algo={algo} {W}x{H} D={D}", flush=True)
+    tiles = ((W + 63) // 64) * ((H + 55) // 56)
+    assert tiles % 8 and tiles * ((D + 63) // 64) >= 1200  # the rule for segments of 64
+    cen = (9, 7) if algo == cs.ALGO_CENSUS else (1, 1)
+    L, R = _pair(W + D, W, H, 0, 9, D - 1)
+    m = cs.Matcher(ctx, W, H, algorithm=algo, window=(7, 7), census=cen, num_disp=D, tol=1)
+    for got, want in zip(m.run(L, R, maps=True), _oracle(algo, L, R, D, (7, 7), cen, 1)):
+        assert np.array_equal(got, want)
+
+
 def test_sad_config0_full(ctx):
     """640x480, D=64, 9x9 SAD, tolerance 1 (the CPU-runnable workload)."""
     L, R = _pair(0, 640, 480, 0, 8, 63)

@@ -63,7 +63,9 @@ sys.path[:0] = [{pkg!r}]
 import clutec_stereo as cs
 ctx = cs.Context(0)
 pairs = [cs.synth_pair(6, 320, 240, 1, 5, 63, 8), cs.synth_pair(5, 320, 240, 0, 8, 63, 8)]
-for algo, win, cen in ((cs.ALGO_CENSUS, (9, 9), (9, 7)), (cs.ALGO_SAD, (7, 7), (1, 1)), (cs.ALGO_AW1, (5, 5), (1, 1))):
+ALGOS = {{"census": (cs.ALGO_CENSUS, (9, 9), (9, 7)), "sad": (cs.ALGO_SAD, (7, 7), (1, 1)),
+         "aw1": (cs.ALGO_AW1, (5, 5), (1, 1)), "ncc": (cs.ALGO_NCC, (9, 9), (1, 1))}}
+for algo, win, cen in [ALGOS[a] for a in {algos!r}]:
     m = None
     for _ in range(2):  # an injected failure may hit the configure
         try:
@@ -83,13 +85,14 @@ for algo, win, cen in ((cs.ALGO_CENSUS, (9, 9), (9, 7)), (cs.ALGO_SAD, (7, 7), (
 """
 
 
-def test_frame_after_an_interrupted_merge_is_clean():
-    """The census, SAD and adaptive-window matchers fold their keys into two planes that
-    every frame's merge clears.  A frame whose merge does not run (a failure injected
+@pytest.mark.parametrize("algos", [["census", "sad", "aw1"], ["ncc"]], ids=lambda a: "-".join(a))
+def test_frame_after_an_interrupted_merge_is_clean(algos):
+    """The census, SAD, adaptive-window and NCC matchers fold their keys into planes that
+    every frame's merge clears (NCC: the right keys).  A frame whose merge does not run (a failure injected
     between the matcher and the merge launch) leaves its keys there; the next frame, on
     another pair, must clear them and equal that pair's frame in a run without failures
     (stale keys of the other pair would win some of its atomicMax and change the maps)."""
-    code = PLANES_CHILD.format(pkg=os.path.join(ROOT, "module.clutec.cuda_amd"))
+    code = PLANES_CHILD.format(pkg=os.path.join(ROOT, "module.clutec.cuda_amd"), algos=algos)
 
     def run(env_extra):
         env = dict(os.environ, **env_extra)
@@ -98,7 +101,7 @@ def test_frame_after_an_interrupted_merge_is_clean():
         return r.stdout.strip().splitlines()
 
     clean = {l.split()[0]: l.split()[-1] for l in run({}) if " ok " in l and " attempt 1 " in l}
-    assert len(clean) == 3
+    assert len(clean) == len(algos)
     checked = set()
     for fail_at in range(1, 60):
         print(f"child with STEREO_FAIL_AT={fail_at}", flush=True)
@@ -112,9 +115,9 @@ def test_frame_after_an_interrupted_merge_is_clean():
                 # the frame after the interrupted one, on the other pair
                 assert nxt and nxt[0].split()[3] == "ok" and nxt[0].split()[-1] == clean[algo], lines
                 checked.add(algo)
-        if len(checked) == 3:
+        if len(checked) == len(algos):
             break
-    assert len(checked) == 3, checked
+    assert len(checked) == len(algos), checked
 
 
 def test_cnn_state_round_trip_resumes_training(ctx):

@@ -44,6 +44,11 @@ def _check(ctx, W, H, D, win, seed, min_agree):
         assert np.all(np.abs(a - b) <= 1e-6)
 
 
+def _short(W, H, D, win):
+    """The rule for the running sums."""
+    return D <= (48 if win >= 9 else 32) and W * H * (2 if win >= 9 else 1) >= 55000 * D
+
+
 @pytest.mark.parametrize("win", [(11, 11), (9, 9), (5, 5)])
 def test_ncc_small(ctx, win):
     _check(ctx, 210, 96, 64, win, 31, 0.999)
@@ -57,9 +62,18 @@ def test_ncc_tall_segments(ctx):
     (65, 33, 8, 11), (64, 32, 8, 5), (127, 35, 24, 7), (128, 37, 32, 9), (129, 34, 40, 11), (161, 33, 64, 11),
     (255, 34, 256, 5), (300, 35, 248, 11), (385, 33, 256, 9), (641, 40, 200, 7)])
 def test_ncc_tiles(ctx, W, H, D, win):
-    """Blocks of 32 x 32 candidates, tiles of 128 columns and 4 or 2 rows, segments of 64 or more
+    """Blocks of 32 x 32 candidates, tiles of 128 columns and 2 rows, segments of 32 or 64
     disparities: one column and row more and less, ranges that end inside a block, images narrower
     than their range."""
+    assert not _short(W, H, D, win) and -(-W // 128) * -(-H // 4) < 1024  # the rule for 2 rows
+    _check(ctx, W, H, D, (win, win), W + D, 0.99)
+
+
+# Tiles of 4 rows, one segment: heights 1 and 2 past a tile, a column past and before one, ranges of 72
+# (blocks up to 96) to 256.
+@pytest.mark.parametrize("W,H,D,win", [(1023, 769, 192, 9), (1025, 770, 72, 11), (897, 514, 104, 7), (1153, 459, 256, 5)])
+def test_ncc_tiles_of_four_rows(ctx, W, H, D, win):
+    assert not _short(W, H, D, win) and -(-W // 128) * -(-H // 4) >= 1024 and H % 4  # the rule
     _check(ctx, W, H, D, (win, win), W + D, 0.99)
 
 
@@ -69,7 +83,7 @@ def test_ncc_tiles(ctx, W, H, D, win):
 def test_ncc_short_ranges(ctx, W, H, D, win):
     """Short ranges of large frames, which take the running sums: ragged tiles of 64 x 52, one group of 8
     disparities, whole and cut statistics tiles of 16, one to three segments."""
-    assert D <= (48 if win >= 9 else 32) and W * H * (2 if win >= 9 else 1) >= 55000 * D  # the rule
+    assert _short(W, H, D, win)
     _check(ctx, W, H, D, (win, win), W + D, 0.99)
 
 

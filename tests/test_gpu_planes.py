@@ -1,4 +1,4 @@
-"""Key planes across frames.  The census / SAD matchers fold every frame's keys into two
+"""Key planes across frames.  The matchers fold every frame's keys into two
 planes with atomicMax, and each frame's merge reads them and clears them for the next
 frame.  Here two different pairs alternate on one driver, so a merge that left keys
 behind, or read another frame's, would change a map: every frame must equal its own
@@ -46,6 +46,24 @@ def test_fused_matcher_planes_across_frames(ctx, algo, window, census):
     want = [_want(algo, L, R, D, window, census) for L, R in pairs]
     assert not np.array_equal(want[0][0], want[1][0])
     m = cs.Matcher(ctx, W, H, algorithm=algo, window=window, census=census, num_disp=D, tol=1)
+    dev = [(cs.DeviceImage.from_array(ctx, L, cs.PIXEL_LUM_U8), cs.DeviceImage.from_array(ctx, R, cs.PIXEL_LUM_U8))
+           for L, R in pairs]
+    _frames(ctx, W, H, lambda k, out, lr, rl: m.process(out, lr, rl, *dev[k]), want)
+
+
+@pytest.mark.parametrize("W,H,D", [(160, 96, 64), (1001, 449, 8)], ids=["matrix", "sums"])
+def test_ncc_planes_across_frames(ctx, W, H, D):
+    """The NCC matcher's right keys meet in a plane that the merge clears; its left keys stay until the next
+    frame writes them.  Each pair's frame must equal the first frame of a new driver."""
+    print(f"NCC planes {W}x{H} D={D}", flush=True)
+    pairs = [cs.synth_pair(s, W, H, 0, 6, 63, 8) for s in (5, 6)]
+
+    def new():
+        return cs.Matcher(ctx, W, H, algorithm=cs.ALGO_NCC, window=(9, 9), num_disp=D, tol=1)
+
+    want = [new().run(L, R, maps=True) for L, R in pairs]
+    assert not np.array_equal(want[0][0], want[1][0])
+    m = new()
     dev = [(cs.DeviceImage.from_array(ctx, L, cs.PIXEL_LUM_U8), cs.DeviceImage.from_array(ctx, R, cs.PIXEL_LUM_U8))
            for L, R in pairs]
     _frames(ctx, W, H, lambda k, out, lr, rl: m.process(out, lr, rl, *dev[k]), want)
