@@ -489,8 +489,11 @@ stereo_status stereo_matcher_configure(stereo_context* ctx, stereo_driver** out,
     }
     if (p->use_disp_input && (st = band_alloc(d))) return cleanup(st);
     // hipMemset returns before the null stream has done it, and a frame may come on a stream that
-    // does not wait for that one
-    if ((e = hipDeviceSynchronize()) != hipSuccess) return cleanup(hip_fail(ctx, e, "hipDeviceSynchronize"));
+    // does not wait for that one.  Waited for by an event: after hipDeviceSynchronize or
+    // hipStreamSynchronize the first frame's launches take longer (rectified 640x480 SAD frame with
+    // its filters: 95 us, 73 so)
+    if ((e = hipEventRecord(d->ev_stop, nullptr)) || (e = hipEventSynchronize(d->ev_stop)))
+        return cleanup(hip_fail(ctx, e, "hipEventSynchronize"));
     *out = d;
     return STEREO_OK;
 }
