@@ -265,47 +265,47 @@ __global__ __launch_bounds__(256) void conv3x3_dw_kernel(CnnDwArgs a)
         __syncthreads();
         // a row past the image has no gradient: its zeros must not meet the rows of X that its taps
         // lie on, which may hold anything
-        const int rows = min(DW_ROWS, a.H - y0);
-        const int nk = SPLIT ? 4 * rows : (wv < rows ? 4 : 0);
-        for (int k = 0; k < nk; ++k) {
-            const int row = SPLIT ? k >> 2 : wv;
-            const int px = 16 * (SPLIT ? k & 3 : k) + 4 * grp;  // this lane's four pixels of the row
-            v4s av[MB];
+        for (int row = SPLIT ? 0 : wv; row < min(DW_ROWS, a.H - y0); row += SPLIT ? 1 : DW_ROWS) {
+#pragma clang loop unroll_count(SPLIT ? 1 : 4)
+            for (int k = 0; k < 4; ++k) {
+                const int px = 16 * k + 4 * grp;  // this lane's four pixels of the row
+                v4s av[MB];
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb) {
-                const uint2 g = *reinterpret_cast<const uint2*>(gs + (co0 + mb * 16 + col) * GS + row * 32 + px / 2);
-                av[mb] = __builtin_bit_cast(v4s, g);
-                bsum[mb] += (bf2f(g.x) + bf2f(g.x >> 16)) + (bf2f(g.y) + bf2f(g.y >> 16));
-            }
-            // pixels past the image: their gradient is 0 and must meet 0, whatever X holds
-            const int in = a.W - (x0 + px);
-            const uint32_t m0 = in >= 2 ? ~0u : (in == 1 ? 0xFFFFu : 0u), m1 = in >= 4 ? ~0u : (in == 3 ? 0xFFFFu : 0u);
-#pragma unroll
-            for (int ky = 0; ky < 3; ++ky)
-#pragma unroll
-                for (int kc = 0; kc < KC; ++kc) {
-                    const uint32_t* src = xs + (ci0 + kc * 16 + col) * XS + (row + ky * DIL) * (DW_PX / 2) + (px + 4) / 2;
-                    uint32_t v[6];  // pixels px - 4 .. px + 7
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        const uint2 q = *reinterpret_cast<const uint2*>(src + 2 * k);
-                        v[2 * k] = q.x;
-                        v[2 * k + 1] = q.y;
-                    }
-#pragma unroll
-                    for (int kx = 0; kx < 3; ++kx) {
-                        constexpr int odd = DIL & 1;
-                        const int s = 4 + (kx - 1) * DIL, w = s >> 1;
-                        const bool shift = kx != 1 && odd;
-                        uint2 x;
-                        x.x = (shift ? __builtin_amdgcn_alignbit(v[w + 1 < 6 ? w + 1 : 5], v[w], 16) : v[w]) & m0;
-                        x.y = (shift ? __builtin_amdgcn_alignbit(v[w + 2 < 6 ? w + 2 : 5], v[w + 1], 16) : v[w + 1]) & m1;
-#pragma unroll
-                        for (int mb = 0; mb < MB; ++mb)
-                            acc[mb][kc][3 * ky + kx] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
-                                av[mb], __builtin_bit_cast(v4s, x), acc[mb][kc][3 * ky + kx], 0, 0, 0);
-                    }
+                for (int mb = 0; mb < MB; ++mb) {
+                    const uint2 g = *reinterpret_cast<const uint2*>(gs + (co0 + mb * 16 + col) * GS + row * 32 + px / 2);
+                    av[mb] = __builtin_bit_cast(v4s, g);
+                    bsum[mb] += (bf2f(g.x) + bf2f(g.x >> 16)) + (bf2f(g.y) + bf2f(g.y >> 16));
                 }
+                // pixels past the image: their gradient is 0 and must meet 0, whatever X holds
+                const int in = a.W - (x0 + px);
+                const uint32_t m0 = in >= 2 ? ~0u : (in == 1 ? 0xFFFFu : 0u), m1 = in >= 4 ? ~0u : (in == 3 ? 0xFFFFu : 0u);
+#pragma unroll
+                for (int ky = 0; ky < 3; ++ky)
+#pragma unroll
+                    for (int kc = 0; kc < KC; ++kc) {
+                        const uint32_t* src = xs + (ci0 + kc * 16 + col) * XS + (row + ky * DIL) * (DW_PX / 2) + (px + 4) / 2;
+                        uint32_t v[6];  // pixels px - 4 .. px + 7
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) {
+                            const uint2 q = *reinterpret_cast<const uint2*>(src + 2 * k);
+                            v[2 * k] = q.x;
+                            v[2 * k + 1] = q.y;
+                        }
+#pragma unroll
+                        for (int kx = 0; kx < 3; ++kx) {
+                            constexpr int odd = DIL & 1;
+                            const int s = 4 + (kx - 1) * DIL, w = s >> 1;
+                            const bool shift = kx != 1 && odd;
+                            uint2 x;
+                            x.x = (shift ? __builtin_amdgcn_alignbit(v[w + 1 < 6 ? w + 1 : 5], v[w], 16) : v[w]) & m0;
+                            x.y = (shift ? __builtin_amdgcn_alignbit(v[w + 2 < 6 ? w + 2 : 5], v[w + 1], 16) : v[w + 1]) & m1;
+#pragma unroll
+                            for (int mb = 0; mb < MB; ++mb)
+                                acc[mb][kc][3 * ky + kx] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                                    av[mb], __builtin_bit_cast(v4s, x), acc[mb][kc][3 * ky + kx], 0, 0, 0);
+                        }
+                    }
+            }
         }
     }
     constexpr int NS = COUT * 9 * CIN + COUT;
