@@ -83,6 +83,8 @@ struct CostSad {
     // 521 -> 507 us)
     static constexpr bool SLIDE = false;
     static constexpr bool PAIRS = true;  // 530 -> 521 us there
+    // asked of the compiler: the batch's default grid is two per CU.  The 154 registers it takes fit
+    // three, which a larger grid then gets
     static constexpr int WG = 2;
     using E = uint8_t;
     using T = uint32_t;

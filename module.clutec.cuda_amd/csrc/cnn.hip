@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void conv3x3_kernel(CnnConvArgs a)
 // What bounds it: the two tensors' bytes (33 MB for 16 frames of 240 x 135 at 16 channels) and
 // the LDS transpose; the MFMAs are 2 % of either.  The form it replaces read every operand
 // from global memory two bytes at a time on one wave per workgroup, 2 waves per CU: 163.8 us
-// at that size, against 20.7 / 23.0 / 28.5 us at dilation 1 / 2 / 4 (the rows of the halo, read
+// at that size, against 20.2 / 22.8 / 28.0 us at dilation 1 / 2 / 4 (the rows of the halo, read
 // by the neighbouring tiles too, grow with the dilation).
 constexpr int DW_ROWS = 4;
 constexpr int DW_PX = 80;  // staged pixels of a row: x0 - 8 .. x0 + 71

@@ -231,8 +231,8 @@ __device__ __forceinline__ uint32_t disparity_bits(int d, int ds, int de, uint32
 // What bounds it: the VALU operations of the key, 8 per candidate (covariance 2, to float and
 // two factors 3, quantise and pack 2, the two maxima 0.5 each), where products and
 // running sums on the VALU took 18.9; the matrix cores are busy a fifth of the time.  1920x1080,
-// 256 disparities, 11 x 11: 411 -> 212 us.  Tiles of 4 rows: with 8 the 2025 workgroups end in a
-// part-filled round (218 us).
+// 256 disparities, 11 x 11: 411 -> 214 us (the frame 429 -> 225).  Tiles of 4 rows: with 8 the 2025
+// workgroups end in a part-filled round (the frame 6 us longer).
 template <int P, bool BAND>
 __global__ __launch_bounds__(256, 3) void ncc_mm_kernel(NccParams p)
 {
