@@ -744,11 +744,16 @@ bool ncc_supported(int ww, int wh, int D)
 // that their two barriers a disparity are hidden (rb = 0).  The matrix kernel costs the same for all
 // ranges up to 32, and more with the window; the running sums hardly see the window.  Whole frames in
 // us, matrix kernel / running sums:
-//                    5x5: D=8      16        24        32        48        64     11x11: 8    16         32         48         64
-//     640 x 480   29.6/29.8  29.8/37.9  29.9/46.8  29.6/42.0  32.3/46.2  31.5/48.7  34.7/29.9  35.1/37.7  34.6/41.9  38.3/47.4  37.0/49.4
-//    1280 x 720   57.6/41.4  57.8/50.9  57.9/61.9  57.2/59.6  66.4/75.9  62.7/83.3  68.7/41.9  69.6/51.8  68.8/60.4  79.1/75.2  75.6/83.7
-//    1920 x 1080  96.2/53.4  96.3/64.8  96.1/79.3  96.0/90.7   114/131    105/132    120/55     120/67     120/92    142/134    132/135
-//    2560 x 1440   158/82     158/100    157/121    156/137    190/209    173/211    198/82     198/101    197/138   235/212    218/214
+//    5x5    D =    8         16         24         32         48         64
+//    640x480   29.6/29.8  29.8/37.9  29.9/46.8  29.6/42.0  32.3/46.2  31.5/48.7
+//   1280x720   57.6/41.4  57.8/50.9  57.9/61.9  57.2/59.6  66.4/75.9  62.7/83.3
+//   1920x1080  96.2/53.4  96.3/64.8  96.1/79.3  96.0/90.7   114/131    105/132
+//   2560x1440   158/82     158/100    157/121    156/137    190/209    173/211
+//   11x11
+//    640x480   34.7/29.9  35.1/37.7  35.1/46.4  34.6/41.9  38.3/47.4  37.0/49.4
+//   1280x720   68.7/41.9  69.6/51.8  69.7/62.9  68.8/60.4  79.1/75.2  75.6/83.7
+//   1920x1080   120/55     120/67     120/82     120/92     142/134    132/135
+//   2560x1440   198/82     198/101    198/124    197/138    235/212    218/214
 // With an initial map the running sums skip what is masked more finely: at 1920 x 1080, a quarter of
 // the size, 11x11, D = 64 150/112, 5x5 119/110; at 1280 x 720 85/67 and 70/65; at 640 x 480 42/51.
 static bool ncc_short_range(int W, int H, int D, int ww, bool band)
